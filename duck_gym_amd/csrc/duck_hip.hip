@@ -284,6 +284,8 @@ class Batch final : public BatchBase {
   void record(hipStream_t s) { hipCheck(hipEventRecord(ready, s), "hipEventRecord"); }
   void launched(const char *what) { hipCheck(hipGetLastError(), what); }
   static int blocks64(int n) { return (n + 63) / 64; }
+  // Blocks of the kernels that give an environment a lane per body slot.
+  static int blocksPerBody(int n) { return (n + 64 / B - 1) / (64 / B); }
   // The float MicroDuck-sized batch has a step compiled without body-pair
   // code, launched for models that have none.
   static constexpr bool kPairless = sizeof(R) == sizeof(float) && L == 16;
@@ -418,7 +420,7 @@ public:
     DeviceGuard guard(device);
     require(bodies && (joints || host.joints.empty()) && diag, "state: null buffer");
     wait(s);
-    snapshotKernel<R, B, J, CG, CS><<<blocks64(count), 64, 0, s>>>(
+    snapshotKernel<R, B, J, CG, CS><<<blocksPerBody(count), 64, 0, s>>>(
         dModel, dStates, blobBytes, count, static_cast<R *>(bodies), static_cast<R *>(joints),
         static_cast<R *>(diag));
     launched("snapshotKernel");
