@@ -150,7 +150,7 @@ template <class R> DeviceModel<R> pack(const HostModel &h, double dt, int iterat
     m.target[j] = R(s.target);
     m.maxTorque[j] = R(s.maxTorque);
   }
-  // Hinge angle of the file state in the batch precision, as resetPose
+  // Hinge angle of the file state in the batch precision, as the reference
   // evaluates it (kernel.cuh:407-412).
   for (int j = 0; j < m.nj; ++j) {
     int a = m.ja[j], b = m.jb[j];
@@ -383,7 +383,7 @@ public:
     const bool noJoints = host.joints.empty();
     require(mask && (q || noJoints) && root, "reset: null buffer");
     wait(s);
-    resetKernel<R, B, J, CG, CS><<<blocks64(count), 64, 0, s>>>(
+    resetKernel<R, B, J, CG, CS><<<blocksPerBody(count), 64, 0, s>>>(
         dModel, dStates, blobBytes, count, mask, static_cast<const R *>(q),
         static_cast<const R *>(root), static_cast<const R *>(ext));
     launched("resetKernel");

@@ -1,7 +1,7 @@
-"""The state snapshot, which gives an environment a lane
+"""The state snapshot and the masked reset, which give an environment a lane
 per body slot (16 or 32): environment counts around a wave's four or two,
-models that fill the slots and models that leave most of them empty, against the
-exported state."""
+models that fill the slots and models that leave most of them empty, against
+the oracle's reset kinematics and snapshot."""
 
 import numpy as np
 import pytest
@@ -25,6 +25,47 @@ def _batch(tmp_path, which, envs, fp64):
     path = tmp_path / "model.duck"
     path.write_text(MODELS[which]())
     return CudaBatch(path, envs, DT, ITER, 0, fp64), Oracle(path, DT, ITER, fp64)
+
+
+def _tolerance(fp64, levels):
+    """A level is one exponential map, three quaternion products and two
+    rotations (about 40 roundings of quantities of order 1)."""
+    return 40 * levels * (2.0 ** -52 if fp64 else 2.0 ** -23)
+
+
+@pytest.mark.parametrize("fp64", [False, True], ids=["fp32", "fp64"])
+@pytest.mark.parametrize("envs", [1, 2, 3, 4, 5, 67])
+@pytest.mark.parametrize("which", sorted(MODELS))
+def test_masked_reset_and_snapshot(tmp_path, which, envs, fp64):
+    batch, oracle = _batch(tmp_path, which, envs, fp64)
+    dtype, J = batch.dtype, batch.num_joints
+    rng = np.random.default_rng(envs)
+    cast = lambda a: torch.tensor(a, dtype=dtype, device=DEV)  # noqa: E731
+    before, state_before = batch.export_state(), batch.state()
+    q, root = rng.uniform(-0.3, 0.3, (envs, J)), rng.uniform(-0.2, 0.2, (envs, 6))
+    mask = rng.uniform(0, 1, envs) < 0.5
+    mask[0] = True
+    bad = envs - 1 if envs > 1 else None
+    if bad is not None:
+        mask[bad] = True
+        root[bad, 3] = np.inf
+    batch.reset(torch.tensor(mask, device=DEV), cast(q), cast(root))
+    bodies, joints, diag = (t.cpu().double().numpy() for t in batch.state())
+    after = batch.export_state()
+    tol = _tolerance(fp64, max(1, J))
+    for e in range(envs):
+        if e == bad:
+            # refused: marked failed, the pose as it was
+            assert diag[e, 5] == 1
+            assert np.array_equal(bodies[e], state_before[0][e].cpu().double().numpy())
+        elif mask[e]:
+            oracle.reset(cast(q).cpu().double().numpy()[e], cast(root).cpu().double().numpy()[e])
+            ob, oj, od = oracle.snapshot()
+            np.testing.assert_allclose(bodies[e], ob, atol=tol, rtol=0)
+            np.testing.assert_allclose(joints[e], oj.reshape(J, 2), atol=tol, rtol=0)
+            assert not diag[e].any()
+        else:
+            assert torch.equal(after[e], before[e])
 
 
 @pytest.mark.parametrize("fp64", [False, True], ids=["fp32", "fp64"])
