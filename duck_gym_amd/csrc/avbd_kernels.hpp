@@ -600,9 +600,9 @@ template <class R> struct ServoArgs {
 // `ctl`) and epilogue (statistics and refresh quantities), defined with the
 // actuator model in avbd_servo.hpp.
 template <class R, int B, int J, int CG, int CS, int L, int JPL, class Env>
-__device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const DeviceModel<R> &M, Env &E,
-                                              int e, int lane, bool valid, int count,
-                                              R (&ctl)[JPL][3]);
+__device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const DeviceModel<R> &M,
+                                              const Frames<R, B, J> &F, Env &E, int e, int lane,
+                                              bool valid, int count, R (&ctl)[JPL][3]);
 template <class R, int B, int J, int CG, int CS, class Env>
 __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const DeviceModel<R> &M, Env &E,
                                               int e);
@@ -783,7 +783,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       massPattern |= (E.s.mass[b] > 0) != (F.mass[b] > 0);
   const bool defaultSchedule = groupOr<L>(massPattern) == 0;
   if constexpr (Servo)
-    servoPrologue<R, B, J, CG, CS, L>(sv, M, E, e, lane, valid, args.count, ctl);
+    servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, valid, args.count, ctl);
 
   // ---- controls (extension.cu:87-110 / kernel.cuh:448-466) ----
   int bad = 0;

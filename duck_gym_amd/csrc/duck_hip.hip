@@ -457,7 +457,7 @@ public:
     DeviceGuard guard(device);
     require(offset && (out || host.joints.empty()), "generalized_loads: null buffer");
     wait(s);
-    generalizedLoadsKernel<R, B, J, CG, CS><<<blocks64(count), 64, 0, s>>>(
+    generalizedLoadsKernel<R, B, J, CG, CS><<<blocksPerBody(count), 64, 0, s>>>(
         dModel, dStates, blobBytes, count, static_cast<const R *>(offset), static_cast<R *>(out));
     launched("generalizedLoadsKernel");
     record(s);

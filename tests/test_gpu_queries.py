@@ -1,7 +1,7 @@
-"""The state snapshot and the masked reset, which give an environment a lane
-per body slot (16 or 32): environment counts around a wave's four or two,
-models that fill the slots and models that leave most of them empty, against
-the oracle's reset kinematics and snapshot."""
+"""The state snapshot, the masked reset and the load query, which give an
+environment a lane per body slot (16 or 32): environment counts around a
+wave's four or two, models that fill the slots and models that leave most of
+them empty, against the oracle's reset kinematics, snapshot and loads."""
 
 import numpy as np
 import pytest
@@ -90,3 +90,35 @@ def test_snapshot_reads_every_field(tmp_path, which, envs, fp64):
         assert np.array_equal(bodies[e], np.concatenate([s["x"], s["q"], s["v"], s["w"]], axis=1))
         want = [s["diag"][0], s["diag"][1], s["diag"][2], s["diag"][3], s["diag"][4], s["failed"]]
         assert np.array_equal(diag[e], np.array(want, bodies.dtype))
+
+
+@pytest.mark.parametrize("fp64", [False, True], ids=["fp32", "fp64"])
+@pytest.mark.parametrize("envs", [1, 5, 67])
+@pytest.mark.parametrize("which", ["microduck", "full"])
+def test_generalized_loads(tmp_path, which, envs, fp64):
+    """Loads after a step (velocities, contacts and drive torques not zero),
+    the oracle's on the same trajectory in float64; in float32 a batch of one
+    environment is the reference (the same code on other lanes)."""
+    batch, oracle = _batch(tmp_path, which, envs, fp64)
+    single, _ = _batch(tmp_path, which, 1, fp64)
+    dtype, J = batch.dtype, batch.num_joints
+    rng = np.random.default_rng(envs)
+    cast = lambda a: torch.tensor(a, dtype=dtype, device=DEV)  # noqa: E731
+    q, root = rng.uniform(-0.1, 0.1, (envs, J)), np.zeros((envs, 6))
+    target, offset = q + rng.uniform(-0.2, 0.2, (envs, J)), rng.uniform(-0.02, 0.02, (envs, 3))
+    force = np.zeros((envs, 3))
+    on = lambda n: torch.ones(n, dtype=torch.bool, device=DEV)  # noqa: E731
+    batch.reset(on(envs), cast(q), cast(root))
+    batch.step(cast(target), cast(force), 2, 8.0, 0.0)
+    loads = batch.generalized_loads(cast(offset))
+    for e in range(envs):
+        if fp64:
+            oracle.reset(q[e], root[e])
+            oracle.step(target[e], force[e], 2, 8.0, 0.0)
+            want = oracle.generalized_loads(offset[e]).reshape(J, 3)
+            scale = max(1.0, np.abs(want).max())
+            np.testing.assert_allclose(loads[e].cpu().numpy(), want, atol=1e-9 * scale, rtol=0)
+        else:
+            single.reset(on(1), cast(q[e:e + 1]), cast(root[e:e + 1]))
+            single.step(cast(target[e:e + 1]), cast(force[:1]), 2, 8.0, 0.0)
+            assert torch.equal(loads[e], single.generalized_loads(cast(offset[e:e + 1]))[0])
