@@ -1,9 +1,9 @@
 // Control-step kernels of the tensor VecEnv (python/duck_gym/tensor_env.py):
 // action clamping and servo targets, and the observation, reward, failure,
 // timeout and episode bookkeeping that the reference assembles from ~40 torch
-// ops per control step (tensor_env.py:178-219, 221-391).  One lane per
-// environment; the root pose and joint state are read straight from the HBM
-// state blob, so no [E,B,13] snapshot is materialised.
+// ops per control step (tensor_env.py:178-219, 221-391).  The root pose and
+// joint state are read straight from the HBM state blob, so no [E,B,13]
+// snapshot is materialised.
 #pragma once
 #include "../../include/duck_hip.h"
 #include "avbd_queries.hpp"
@@ -131,138 +131,216 @@ struct TaskBuffers {
   void *diag;                // [E,6] R, may be null
 };
 
-// What the task kernel reads of a blob, staged in LDS: the 16-byte chunks
-// covering the diagnostics through the angular velocities (the targets, force
-// and the body poses and velocities lie between them).  A workgroup of 64
-// lanes copies its environments' ranges with whole-wave loads (each
-// environment's chunks are consecutive, so a load instruction covers a few
-// cache lines instead of one line per lane), then each lane computes one
-// environment from LDS.
-template <class S> constexpr size_t taskStageBegin() { return diagBegin<S>() / 16 * 16; }
-template <class S> constexpr size_t taskStageEnd() { return (offsetof(S, w) + sizeof(S::w) + 15) / 16 * 16; }
-template <class S> constexpr int taskStageChunks() { return int((taskStageEnd<S>() - taskStageBegin<S>()) / 16); }
-// environments per workgroup: as many as 60 KiB of LDS holds, at most 64; the
-// record stride in words is the chunks' plus one (odd: the lanes' records
-// fall on distinct LDS banks) for a float batch, plus two for a double one
-// (whole 8-byte words)
-template <class S> constexpr int taskStageStride() {
-  return 4 * taskStageChunks<S>() + (sizeof(S::diag[0]) == 4 ? 1 : 2);
-}
-template <class S> constexpr int taskEnvsPerBlock() {
-  return 61440 / (4 * taskStageStride<S>()) > 64 ? 64 : 61440 / (4 * taskStageStride<S>());
-}
-
-// The staged fields of one environment (the same values as the blob's).
-template <class R, int B, int J, int CG, int CS> struct TaskStage {
-  using State = EnvState<R, B, J, CG, CS>;
-  const DeviceModel<R> &M;
-  const R *r; // the environment's staged words, from taskStageBegin
-  static constexpr int at(size_t offset) { return int((offset - taskStageBegin<State>()) / sizeof(R)); }
-  DUCK_HD R x(int k, int b) const { return r[at(offsetof(State, x)) + k * B + b]; }
-  DUCK_HD R q(int k, int b) const { return r[at(offsetof(State, q)) + k * B + b]; }
-  DUCK_HD R v(int k, int b) const { return r[at(offsetof(State, v)) + k * B + b]; }
-  DUCK_HD R w(int k, int b) const { return r[at(offsetof(State, w)) + k * B + b]; }
-  DUCK_HD R diag(int k) const { return r[at(offsetof(State, diag)) + k]; }
-  DUCK_HD Q4<R> Q(int b) const { return {q(0, b), q(1, b), q(2, b), q(3, b)}; }
-  DUCK_HD V3<R> W(int b) const { return {w(0, b), w(1, b), w(2, b)}; }
-  DUCK_HD V3<R> mv(const R (&a)[3][kMaxModelJoints], int j) const { return {a[0][j], a[1][j], a[2][j]}; }
-  DUCK_HD R angle(int j) const {
-    return hingeAngle(Q(M.ja[j]), Q(M.jb[j]), mv(M.axisA, j), mv(M.tangentA, j), mv(M.tangentB, j));
-  }
-};
-
+// The task step and observation of [E] environments in one launch.  A wave
+// takes 64 / B environments with B lanes each: lane b reads its body's
+// component rows (and checks them finite), lane j forms hinge j's angle, rate,
+// action terms and observation entries, lanes 0 to 2 add the three sums over
+// the hinges in hinge order, lanes 0 and 1 form the two feet's terms, and
+// every lane of an environment evaluates the root frame and the reward (one
+// instruction stream either way); the observation rows leave as one contiguous
+// run.  Every value is formed by the operations, in the order, of one lane
+// going over the environment.  Bound by a few dependent chains and memory
+// round trips: 7.4 us at 4096 environments, 16 us at 32768.  A lane per
+// environment (64 waves at 4096, each hinge after the other) took 26 and
+// 27 us.
 template <class R, int B, int J, int CG, int CS>
 __global__ __launch_bounds__(64) void taskKernel(DuckTask t, int mode, const DeviceModel<R> *model,
                                                  unsigned char *states, long long blobBytes, int count,
                                                  TaskBuffers io) {
+  static_assert(J <= B && 64 % B == 0 && B >= 6, "a lane per body, hinge and diagnostic");
   using State = EnvState<R, B, J, CG, CS>;
-  constexpr int CH = taskStageChunks<State>(), STRIDE = taskStageStride<State>(),
-                TE = taskEnvsPerBlock<State>();
-  static_assert(TE >= 1 && (4 * STRIDE) % sizeof(R) == 0 && taskStageBegin<State>() % sizeof(R) == 0,
-                "a staged record holds whole words of the batch dtype");
-  __shared__ unsigned stage[TE * STRIDE];
-  const int e0 = blockIdx.x * TE;
-  const int n = count - e0 < TE ? count - e0 : TE;
-  // chunk c of environment i is item i CH + c; the lanes take the items in
-  // turn, so that a lane's loads are independent and in flight together
-#pragma unroll 8
-  for (int item = threadIdx.x; item < n * CH; item += 64) {
-    const int i = item / CH, c = item - i * CH;
-    const uint4 v = reinterpret_cast<const uint4 *>(states + blobBytes * (e0 + i) + taskStageBegin<State>())[c];
-    unsigned *dst = stage + i * STRIDE + 4 * c;
-    dst[0] = v.x;
-    dst[1] = v.y;
-    dst[2] = v.z;
-    dst[3] = v.w;
-  }
-  __syncthreads();
-  const int e = e0 + int(threadIdx.x);
-  if (threadIdx.x >= TE || e >= count)
-    return;
+  constexpr int G = 64 / B, D = 18 + 3 * J; // the widest observation row
+  __shared__ R stage[G][13][B];             // x, q, v, w rows
+  __shared__ R terms[G][3][J], sums[G][3], feet[G][2][2];
+  __shared__ R contactZ[G][CG + CS];
+  __shared__ int contactId[G][CG + CS];
+  __shared__ float rows[G * D];
   const DeviceModel<R> &M = *model;
-  const State &s = blobAt<State>(states, blobBytes, e);
-  const TaskStage<R, B, J, CG, CS> view{M, reinterpret_cast<const R *>(stage + threadIdx.x * STRIDE)};
-  const int nj = M.nj;
-  R *act = static_cast<R *>(io.action) + size_t(e) * nj;
-  R *last = static_cast<R *>(io.lastAction) + size_t(e) * nj;
-  R *filt = io.filtered ? static_cast<R *>(io.filtered) + size_t(e) * 2 : nullptr;
-  const R *cmd = io.commands ? static_cast<const R *>(io.commands) + size_t(e) * 2 : nullptr;
+  const int lane = threadIdx.x % B, g = threadIdx.x / B;
+  const int e0 = blockIdx.x * G, e = e0 + g, n = count - e0 < G ? count - e0 : G;
+  const bool valid = e < count, step = mode == kTaskStep;
+  const int nb = M.nb, nj = M.nj, width = taskObsDim(t, nj);
+  const State &s = blobAt<State>(states, blobBytes, valid ? e : 0);
+  const size_t row = size_t(valid ? e : 0), at = row * nj + lane;
+  const bool joint = valid && lane < nj;
+  R *actions = static_cast<R *>(io.action), *lasts = static_cast<R *>(io.lastAction);
+  R *filt = io.filtered ? static_cast<R *>(io.filtered) + row * 2 : nullptr;
 
-  if (mode == kTaskReset && io.mask && io.mask[e]) {
+  // the hinge's frames, the body's rows and the caller's values
+  const int jc = lane < nj ? lane : 0, ja = M.ja[jc], jb = M.jb[jc];
+  const V3<R> axisA{M.axisA[0][jc], M.axisA[1][jc], M.axisA[2][jc]};
+  const V3<R> tangentA{M.tangentA[0][jc], M.tangentA[1][jc], M.tangentA[2][jc]};
+  const V3<R> tangentB{M.tangentB[0][jc], M.tangentB[1][jc], M.tangentB[2][jc]};
+  const R home = R(t.home[jc]);
+  bool finite = true;
+  if (valid && lane < nb) {
+    const R body[13] = {s.x[0][lane], s.x[1][lane], s.x[2][lane], s.q[0][lane], s.q[1][lane],
+                        s.q[2][lane], s.q[3][lane], s.v[0][lane], s.v[1][lane], s.v[2][lane],
+                        s.w[0][lane], s.w[1][lane], s.w[2][lane]};
+#pragma unroll
+    for (int k = 0; k < 13; ++k) {
+      finite = finite && mfinite(body[k]);
+      stage[g][k][lane] = body[k];
+    }
+  }
+  const bool restart = valid && !step && io.mask && io.mask[row] != 0;
+  R act = joint && !restart ? actions[at] : R(0);
+  const R last = joint && step ? lasts[at] : R(0);
+  R cmd[2] = {0, 0}, filtered[2] = {0, 0}, diag[6] = {0, 0, 0, 0, 0, 0};
+  if (valid && io.commands) {
+    cmd[0] = static_cast<const R *>(io.commands)[row * 2];
+    cmd[1] = static_cast<const R *>(io.commands)[row * 2 + 1];
+  }
+  if (valid && filt && !restart) {
+    filtered[0] = filt[0];
+    filtered[1] = filt[1];
+  }
+  long long episode = valid && !restart ? io.episode[row] : 0;
+  const float returns = valid && step ? io.returns[row] : 0.f;
+  if (valid && step) {
+    constexpr int slot[5] = {kJointError, kPenetration, kContacts, kConverged, kAxisError};
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+      diag[k] = s.diag[slot[k]];
+    diag[5] = R(s.failed);
+  }
+  if (restart) {
     // tensor_env.py:199-203: restart the episode bookkeeping of reset envs.
-    for (int j = 0; j < nj; ++j)
-      act[j] = R(0);
-    if (filt)
-      filt[0] = filt[1] = R(0);
-    if (io.forces)
-      for (int k = 0; k < 3; ++k)
-        static_cast<R *>(io.forces)[size_t(e) * 3 + k] = R(0);
-    io.episode[e] = 0;
-    io.returns[e] = 0.f;
+    if (joint)
+      actions[at] = R(0);
+    if (lane < 2 && filt)
+      filt[lane] = R(0);
+    if (lane < 3 && io.forces)
+      static_cast<R *>(io.forces)[row * 3 + lane] = R(0);
+    if (lane == 0) {
+      io.episode[row] = 0;
+      io.returns[row] = 0.f;
+    }
+  }
+  const int ngc = valid ? (s.ngc < CG ? s.ngc : CG) : 0, nsc = valid ? (s.nsc < CS ? s.nsc : CS) : 0;
+  if (step && t.load_transfer) {
+    // z of contactForcesKernel's term of each contact
+    for (int i = lane; i < ngc; i += B) {
+      const auto &c = s.gc[i];
+      contactId[g][i] = c.id;
+      contactZ[g][i] = (-((V3<R>{1, 0, 0} * c.lambda[0] + V3<R>{0, 1, 0} * c.lambda[1]) +
+                          V3<R>{0, 0, 1} * c.lambda[2]))
+                           .z;
+    }
+    for (int i = lane; i < nsc; i += B) {
+      contactId[g][CG + i] = s.sc[i].id;
+      contactZ[g][CG + i] = (-selfForceWorld(s.sc[i])).z;
+    }
+  }
+  const uint64_t group = ((uint64_t(1) << B) - 1) << (g * B);
+  finite = (__ballot(!finite) & group) == 0;
+  __syncthreads();
+
+  auto Q = [&](int b) { return Q4<R>{stage[g][3][b], stage[g][4][b], stage[g][5][b], stage[g][6][b]}; };
+  auto X = [&](int b) { return V3<R>{stage[g][0][b], stage[g][1][b], stage[g][2][b]}; };
+  auto W = [&](int b) { return V3<R>{stage[g][10][b], stage[g][11][b], stage[g][12][b]}; };
+  float *o = rows + g * width;
+  const int heads = t.kind == DUCK_TASK_ROLLOUT ? 6 : 10;
+  if (joint) {
+    const Q4<R> qa = Q(ja), qb = Q(jb);
+    const R d = hingeAngle(qa, qb, axisA, tangentA, tangentB) - home;
+    const R rate = dot(W(jb) - W(ja), rotate(qa, axisA));
+    const R da = act - last;
+    terms[g][0][lane] = d * d;
+    terms[g][1][lane] = act * act;
+    terms[g][2][lane] = da * da;
+    o[heads + lane] = float(d);
+    o[heads + nj + lane] = float(R(0.1) * rate);
+    o[heads + 2 * nj + lane] = float(act);
   }
 
   // Root frame q = q_body1 (x) conj(root_iquat) (tensor_env.py:140-142, 222).
   const int root = 1;
-  Q4<R> qb = view.Q(root);
-  Q4<R> iq{R(t.iquat[0]), -R(t.iquat[1]), -R(t.iquat[2]), -R(t.iquat[3])};
-  Q4<R> q = qb * iq;
-  V3<R> g = rotateInv(q, V3<R>{R(0), R(0), R(-1)});
-  V3<R> vel{view.v(0, root), view.v(1, root), view.v(2, root)};
-  V3<R> v = rotateInv(q, vel);
-  V3<R> w = rotateInv(q, view.W(root));
-  R yawC = R(1) - R(2) * (q.y * q.y + q.z * q.z);
-  R yawS = R(2) * (q.w * q.z + q.x * q.y);
-  R height = view.x(2, root) - R(t.root_height);
+  const Q4<R> iq{R(t.iquat[0]), -R(t.iquat[1]), -R(t.iquat[2]), -R(t.iquat[3])};
+  const Q4<R> q = Q(root) * iq;
+  const V3<R> grav = rotateInv(q, V3<R>{R(0), R(0), R(-1)});
+  const V3<R> vel{stage[g][7][root], stage[g][8][root], stage[g][9][root]};
+  const V3<R> v = rotateInv(q, vel);
+  const V3<R> w = rotateInv(q, W(root));
+  const R yawC = R(1) - R(2) * (q.y * q.y + q.z * q.z);
+  const R yawS = R(2) * (q.w * q.z + q.x * q.y);
+  const R height = X(root).z - R(t.root_height);
 
-  R reward = 0;
-  bool failed = false, timeout = false;
-  if (mode == kTaskStep) {
+  if (step && valid && lane < 2) {
+    // Gait shaping (tensor_env.py:328-354), at the counter after this step:
+    // lane f forms foot f's squared gap and load error.
+    const int f = lane, fb = t.feet[f];
+    if (t.foot_clearance) {
+      // the feet's lowest collision points against a lift that peaks
+      // mid-swing; the phase is float32 (an int64 counter times a float)
+      const R *pts = static_cast<const R *>(t.foot_point);
+      const V3<R> p = X(fb);
+      const Q4<R> qf = Q(fb);
+      // inverse_rotate(q, up) (tensor_env.py:21-23)
+      const V3<R> up{R(0), R(0), R(1)}, u{-qf.x, -qf.y, -qf.z};
+      const V3<R> tt = cross(u, up) * R(2);
+      const V3<R> localUp = (up + tt * qf.w) + cross(u, tt);
+      R lowest = R(0);
+      for (int k = 0; k < t.foot_points; ++k) {
+        const R *c = pts + (size_t(f) * t.foot_points + k) * 3;
+        const R h = (c[0] * localUp.x + c[1] * localUp.y + c[2] * localUp.z) + p.z;
+        lowest = k == 0 || h < lowest ? h : lowest;
+      }
+      float phase =
+          float(episode + 1) * float(t.control_dt) / float(t.gait_period) + (f ? 0.5f : 0.0f);
+      phase = fmodf(phase, 1.0f);
+      float swing = (phase - 0.6f) / 0.4f;
+      swing = swing < 0.0f ? 0.0f : (swing > 1.0f ? 1.0f : swing);
+      const float sw = sinf(float(3.14159265358979323846) * swing);
+      const R desired = R(float(t.gait_lift) * (sw * sw));
+      const R gap = (lowest < R(0) ? R(0) : lowest) - desired;
+      feet[g][0][f] = gap * gap;
+    }
+    if (t.load_transfer) {
+      // vertical contact force of each foot, in body weights, against a
+      // sinusoidal left/right split
+      const R cycle = (R(episode) + R(1)) * R(t.control_dt) / R(t.gait_period);
+      const R left = R(0.5) + R(0.5) * tsin(R(2 * 3.14159265358979323846) * (cycle - R(0.05)));
+      R z = 0;
+      for (int i = 0; i < ngc; ++i)
+        if (gcBody(contactId[g][i]) == fb)
+          z += contactZ[g][i];
+      for (int i = 0; i < nsc; ++i) {
+        const int id = contactId[g][CG + i];
+        const R fz = contactZ[g][CG + i];
+        if (scBody(id) == fb)
+          z += fz;
+        if (scOther(id) == fb)
+          z -= fz;
+      }
+      R force = z / R(t.weight);
+      force = force < R(0) ? R(0) : (force > R(3) ? R(3) : force);
+      const R d = force - (f ? R(1) - left : left);
+      feet[g][1][f] = d * d;
+    }
+  }
+  __syncthreads();
+  if (step && valid && lane < 3) {
+    R sum = 0;
+    for (int j = 0; j < nj; ++j)
+      sum += terms[g][lane][j];
+    sums[g][lane] = sum;
+  }
+  __syncthreads();
+  if (step) {
     // Failure (tensor_env.py:294-301; the rollout task fails on a fall).
-    bool finite = true;
-    for (int b = 0; b < M.nb; ++b) {
-      for (int k = 0; k < 3; ++k)
-        finite = finite && mfinite(view.x(k, b)) && mfinite(view.v(k, b)) && mfinite(view.w(k, b));
-      for (int k = 0; k < 4; ++k)
-        finite = finite && mfinite(view.q(k, b));
-    }
     const R cosHalf = R(cosf(0.5f)); // torch.cos of a float32 0.5
+    bool failed;
     if (t.kind == DUCK_TASK_ROLLOUT)
-      failed = view.x(2, root) < R(t.fall_height);
+      failed = X(root).z < R(t.fall_height);
     else
-      failed = g.z > -cosHalf || mabs(height) > R(0.04) || view.diag(kJointError) > R(0.005) ||
-               view.diag(kPenetration) > R(0.005);
-    failed = failed || s.failed > 0 || !finite;
+      failed = grav.z > -cosHalf || mabs(height) > R(0.04) || diag[0] > R(0.005) || diag[1] > R(0.005);
+    failed = failed || diag[5] > R(0) || !finite;
 
-    R pose = 0, act2 = 0, dact2 = 0;
-    for (int j = 0; j < nj; ++j) {
-      R d = view.angle(j) - R(t.home[j]);
-      pose += d * d;
-      act2 += act[j] * act[j];
-      R da = act[j] - last[j];
-      dact2 += da * da;
-    }
-    R tilt = g.x * g.x + g.y * g.y;
-    R w2 = dot(w, w);
+    const R pose = sums[g][0], act2 = sums[g][1], dact2 = sums[g][2];
+    const R tilt = grav.x * grav.x + grav.y * grav.y;
+    const R w2 = dot(w, w);
+    R reward;
     if (t.kind == DUCK_TASK_STANDING) {
       // tensor_env.py:302-310
       reward = R(1.5) * mexp(R(-20) * tilt) + mexp(R(-2000) * height * height) +
@@ -272,128 +350,83 @@ __global__ __launch_bounds__(64) void taskKernel(DuckTask t, int mode, const Dev
       // tensor_env.py:311-327: world-frame COM velocity against the command.
       R vx = vel.x, vy = vel.y;
       if (t.kind == DUCK_TASK_LOCOMOTION && t.velocity_filter) {
-        R alpha = R(t.velocity_alpha);
-        filt[0] = (R(1) - alpha) * filt[0] + alpha * vx;
-        filt[1] = (R(1) - alpha) * filt[1] + alpha * vy;
-        vx = filt[0];
-        vy = filt[1];
+        const R alpha = R(t.velocity_alpha);
+        filtered[0] = (R(1) - alpha) * filtered[0] + alpha * vx;
+        filtered[1] = (R(1) - alpha) * filtered[1] + alpha * vy;
+        vx = filtered[0];
+        vy = filtered[1];
       }
-      R ex = vx - cmd[0], ey = vy - cmd[1];
-      R error = ex * ex + ey * ey;
-      R sigma = R(t.tracking_sigma);
+      const R ex = vx - cmd[0], ey = vy - cmd[1];
+      const R error = ex * ex + ey * ey;
+      const R sigma = R(t.tracking_sigma);
       reward = R(1) * mexp(R(-20) * tilt) + mexp(R(-2000) * height * height) +
                R(t.tracking_weight) * mexp(-error / (sigma * sigma)) - R(0.1) * w2 -
                R(t.heading_weight) * (R(1) - yawC) - R(0.02) * act2 - R(0.03) * dact2;
     }
-    // Gait shaping (tensor_env.py:328-354), at the counter after this step.
-    const long long next = io.episode[e] + 1;
-    if (t.foot_clearance) {
-      // the feet's lowest collision points against a lift that peaks
-      // mid-swing; the phase is float32 (an int64 counter times a float)
-      const R *pts = static_cast<const R *>(t.foot_point);
-      R penalty = 0;
-      for (int f = 0; f < 2; ++f) {
-        const int fb = t.feet[f];
-        const V3<R> p{view.x(0, fb), view.x(1, fb), view.x(2, fb)};
-        const Q4<R> qf = view.Q(fb);
-        // inverse_rotate(q, up) (tensor_env.py:21-23)
-        const V3<R> up{R(0), R(0), R(1)}, u{-qf.x, -qf.y, -qf.z};
-        const V3<R> tt = cross(u, up) * R(2);
-        const V3<R> localUp = (up + tt * qf.w) + cross(u, tt);
-        R lowest = R(0);
-        for (int k = 0; k < t.foot_points; ++k) {
-          const R *v = pts + (size_t(f) * t.foot_points + k) * 3;
-          const R h = (v[0] * localUp.x + v[1] * localUp.y + v[2] * localUp.z) + p.z;
-          lowest = k == 0 || h < lowest ? h : lowest;
-        }
-        float phase = float(next) * float(t.control_dt) / float(t.gait_period) + (f ? 0.5f : 0.0f);
-        phase = fmodf(phase, 1.0f);
-        float swing = (phase - 0.6f) / 0.4f;
-        swing = swing < 0.0f ? 0.0f : (swing > 1.0f ? 1.0f : swing);
-        const float sw = sinf(float(3.14159265358979323846) * swing);
-        const R desired = R(float(t.gait_lift) * (sw * sw));
-        const R gap = (lowest < R(0) ? R(0) : lowest) - desired;
-        penalty += gap * gap;
-      }
-      reward -= R(20000) * penalty;
-    }
-    if (t.load_transfer) {
-      // vertical contact force of each foot, in body weights, against a
-      // sinusoidal left/right split
-      const R cycle = (R(io.episode[e]) + R(1)) * R(t.control_dt) / R(t.gait_period);
-      const R left = R(0.5) + R(0.5) * tsin(R(2 * 3.14159265358979323846) * (cycle - R(0.05)));
-      R penalty = 0;
-      for (int f = 0; f < 2; ++f) {
-        R force = contactForceZ(s, t.feet[f]) / R(t.weight);
-        force = force < R(0) ? R(0) : (force > R(3) ? R(3) : force);
-        const R d = force - (f ? R(1) - left : left);
-        penalty += d * d;
-      }
-      reward -= R(3) * penalty;
-    }
+    if (t.foot_clearance)
+      reward -= R(20000) * (feet[g][0][0] + feet[g][0][1]);
+    if (t.load_transfer)
+      reward -= R(3) * (feet[g][1][0] + feet[g][1][1]);
     reward = (failed ? R(-2) : reward) * R(t.control_dt);
-    long long ep = next;
-    io.episode[e] = ep;
-    io.returns[e] += float(reward);
-    timeout = ep >= t.max_episode_length && !failed;
-    io.reward[e] = float(reward);
-    io.failed[e] = failed;
-    io.timeout[e] = timeout;
-    io.done[e] = failed || timeout;
-    for (int j = 0; j < nj; ++j)
-      last[j] = act[j];
-    if (io.diag) {
-      R *d = static_cast<R *>(io.diag) + size_t(e) * 6;
-      d[0] = view.diag(kJointError);
-      d[1] = view.diag(kPenetration);
-      d[2] = view.diag(kContacts);
-      d[3] = view.diag(kConverged);
-      d[4] = view.diag(kAxisError);
-      d[5] = R(s.failed);
+    episode += 1;
+    const bool timeout = episode >= t.max_episode_length && !failed;
+    if (joint)
+      lasts[at] = act;
+    if (valid && lane == 0) {
+      io.episode[row] = episode;
+      io.returns[row] = returns + float(reward);
+      io.reward[row] = float(reward);
+      io.failed[row] = failed;
+      io.timeout[row] = timeout;
+      io.done[row] = failed || timeout;
+      if (t.kind == DUCK_TASK_LOCOMOTION && t.velocity_filter) {
+        filt[0] = filtered[0];
+        filt[1] = filtered[1];
+      }
+    }
+    if (valid && io.diag) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+        if (lane == k)
+          static_cast<R *>(io.diag)[row * 6 + k] = diag[k];
     }
   }
 
-  // Observation (tensor_env.py:238-258), cast to float32.
-  float *o = io.obs + size_t(e) * taskObsDim(t, nj);
-  int k = 0;
-  o[k++] = float(g.x);
-  o[k++] = float(g.y);
-  o[k++] = float(g.z);
-  if (t.kind != DUCK_TASK_ROLLOUT) {
-    o[k++] = float(v.x);
-    o[k++] = float(v.y);
-    o[k++] = float(v.z);
-  }
-  o[k++] = float(w.x);
-  o[k++] = float(w.y);
-  o[k++] = float(w.z);
-  if (t.kind != DUCK_TASK_ROLLOUT)
-    o[k++] = float(height);
-  for (int j = 0; j < nj; ++j)
-    o[k + j] = float(view.angle(j) - R(t.home[j]));
-  k += nj;
-  for (int j = 0; j < nj; ++j) {
-    R rate = dot(view.W(M.jb[j]) - view.W(M.ja[j]), rotate(view.Q(M.ja[j]), view.mv(M.axisA, j)));
-    o[k + j] = float(R(0.1) * rate);
-  }
-  k += nj;
-  for (int j = 0; j < nj; ++j)
-    o[k + j] = float(act[j]);
-  k += nj;
-  if (t.kind == DUCK_TASK_LOCOMOTION) {
-    // (episode * control_dt) * (2 pi / period), the factor formed in double.
-    R phase = R(io.episode[e]) * R(t.control_dt) * R(2 * 3.14159265358979323846 / t.gait_period);
-    o[k++] = float(cmd[0]);
-    o[k++] = float(cmd[1]);
-    o[k++] = float(yawC);
-    o[k++] = float(yawS);
-    o[k++] = float(msin(phase));
-    o[k++] = float(mcos(phase));
-    if (t.velocity_filter) {
-      o[k++] = float(filt[0]);
-      o[k++] = float(filt[1]);
+  // Observation (tensor_env.py:238-258), cast to float32: the entries before
+  // and after the hinges'.
+  if (valid && lane == 0) {
+    int k = 0;
+    o[k++] = float(grav.x);
+    o[k++] = float(grav.y);
+    o[k++] = float(grav.z);
+    if (t.kind != DUCK_TASK_ROLLOUT) {
+      o[k++] = float(v.x);
+      o[k++] = float(v.y);
+      o[k++] = float(v.z);
+    }
+    o[k++] = float(w.x);
+    o[k++] = float(w.y);
+    o[k++] = float(w.z);
+    if (t.kind != DUCK_TASK_ROLLOUT)
+      o[k++] = float(height);
+    k += 3 * nj;
+    if (t.kind == DUCK_TASK_LOCOMOTION) {
+      // (episode * control_dt) * (2 pi / period), the factor formed in double.
+      const R phase = R(episode) * R(t.control_dt) * R(2 * 3.14159265358979323846 / t.gait_period);
+      o[k++] = float(cmd[0]);
+      o[k++] = float(cmd[1]);
+      o[k++] = float(yawC);
+      o[k++] = float(yawS);
+      o[k++] = float(msin(phase));
+      o[k++] = float(mcos(phase));
+      if (t.velocity_filter) {
+        o[k++] = float(filtered[0]);
+        o[k++] = float(filtered[1]);
+      }
     }
   }
+  __syncthreads();
+  copyRows(io.obs + size_t(e0) * width, rows, n * width, threadIdx.x);
 }
 
 } // namespace duckhip

@@ -225,3 +225,15 @@ def test_observations_from_state_equal_the_kernel(model_dir, task, kw):
         kernel_rows, _ = env.get_observations()
         assert torch_rows.shape == kernel_rows.shape
         np.testing.assert_allclose(_np(torch_rows), _np(kernel_rows), rtol=1e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("envs", [1, 3, 5, 67])
+@pytest.mark.parametrize("task,kind", [("standing", T.STANDING), ("locomotion", T.LOCOMOTION),
+                                       ("rollout", T.ROLLOUT)])
+def test_env_counts_around_a_wave(model_dir, task, kind, envs):
+    """A wave of the task launch takes four environments: counts that leave
+    it partly empty."""
+    env = TensorEnv(model_dir, envs, ITER, DT, 2, seed=3, task=task, auto_reset=False)
+    gen = torch.Generator(device=DEV).manual_seed(envs)
+    for _ in range(2):
+        _check_step(env, kind, torch.rand(envs, 14, generator=gen, device=DEV) * 2.4 - 1.2, 1e-5)
