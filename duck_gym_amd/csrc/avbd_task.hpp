@@ -429,4 +429,76 @@ __global__ __launch_bounds__(64) void taskKernel(DuckTask t, int mode, const Dev
   copyRows(io.obs + size_t(e0) * width, rows, n * width, threadIdx.x);
 }
 
+// The maximum of the two, NaN when either is (torch.amax).
+template <class R> DUCK_HD R maxNan(R a, R b) { return a != a || b != b ? R(NAN) : (a > b ? a : b); }
+
+// Sums (or, for the logged maxima, maxima) over the wave, on every lane.
+constexpr int kTaskLogs = DUCK_TASK_LOGS;
+template <class R> __device__ __forceinline__ void waveLogs(R (&v)[kTaskLogs]) {
+#pragma unroll
+  for (int o = 32; o > 0; o /= 2)
+#pragma unroll
+    for (int k = 0; k < kTaskLogs; ++k) {
+      const R u = __shfl_xor(v[k], o, 64);
+      v[k] = k == 1 || k == 2 ? maxNan(v[k], u) : v[k] + u;
+    }
+}
+
+// The scalars that tensor_env.py:367-391 logs after a step, over all
+// environments, in two launches: here a wave of 64 environments forms its
+// terms (the root's pose and velocity straight from the blobs) and their sums
+// and maxima as row 1 + block of `out`; taskLogReduceKernel folds the rows
+// into row 0 in row order, so the values do not depend on timing.  Bound by
+// launch: 2 x 4 us at 4096 environments in the place of a state snapshot and
+// some 50 torch launches (about 190 us of them on the stream).
+template <class R, int B, int J, int CG, int CS>
+__global__ __launch_bounds__(64) void taskLogKernel(DuckTask t, unsigned char *states, long long blobBytes,
+                                                    int count, const unsigned char *failed, const R *diag,
+                                                    const R *commands, const R *filtered, R speed,
+                                                    R *out) {
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  const bool valid = e < count;
+  R v[kTaskLogs] = {0, R(-INFINITY), R(-INFINITY), 0, 0, 0, 0};
+  if (valid) {
+    v[0] = failed[e] ? R(1) : R(0);
+    v[1] = diag[size_t(e) * 6];
+    v[2] = diag[size_t(e) * 6 + 1];
+  }
+  if (valid && t.kind == DUCK_TASK_LOCOMOTION) {
+    const auto &s = blobAt<EnvState<R, B, J, CG, CS>>(states, blobBytes, e);
+    const Q4<R> q = Q4<R>{s.q[0][1], s.q[1][1], s.q[2][1], s.q[3][1]} *
+                    Q4<R>{R(t.iquat[0]), -R(t.iquat[1]), -R(t.iquat[2]), -R(t.iquat[3])};
+    const R vx = s.v[0][1], vy = s.v[1][1];
+    const R cx = commands[size_t(e) * 2], cy = commands[size_t(e) * 2 + 1];
+    const R fx = (t.velocity_filter ? filtered[size_t(e) * 2] : vx) - cx;
+    const R fy = (t.velocity_filter ? filtered[size_t(e) * 2 + 1] : vy) - cy;
+    const R dx = vx - cx, dy = vy - cy;
+    v[3] = msqrt(dx * dx + dy * dy);
+    v[4] = vx * (cx / speed) + vy * (cy / speed);
+    v[5] = msqrt(fx * fx + fy * fy);
+    v[6] = mabs(matan2(R(2) * (q.w * q.z + q.x * q.y), R(1) - R(2) * (q.y * q.y + q.z * q.z)));
+  }
+  waveLogs(v);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < kTaskLogs; ++k)
+      out[(1 + size_t(blockIdx.x)) * kTaskLogs + k] = v[k];
+}
+
+template <class R>
+__global__ __launch_bounds__(64) void taskLogReduceKernel(int rows, int count, R *out) {
+  R v[kTaskLogs] = {0, R(-INFINITY), R(-INFINITY), 0, 0, 0, 0};
+  for (int r = threadIdx.x; r < rows; r += 64)
+#pragma unroll
+    for (int k = 0; k < kTaskLogs; ++k) {
+      const R u = out[(1 + size_t(r)) * kTaskLogs + k];
+      v[k] = k == 1 || k == 2 ? maxNan(v[k], u) : v[k] + u;
+    }
+  waveLogs(v);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < kTaskLogs; ++k)
+      out[k] = k == 1 || k == 2 ? v[k] : v[k] / R(count);
+}
+
 } // namespace duckhip

@@ -260,6 +260,8 @@ struct BatchBase {
   virtual void taskResetInputs(const DuckTask &, const unsigned char *, const void *, const void *,
                                const long long *, int, double, const void *, void *, void *,
                                void *, hipStream_t) = 0;
+  virtual void taskLog(const DuckTask &, const unsigned char *, const void *, const void *,
+                       const void *, double, void *, hipStream_t) = 0;
   virtual void servo(const DuckServo &, const ServoBuffers &, hipStream_t) = 0;
   virtual void servoSubstep(const DuckServo &, const DuckServoSubstep &, hipStream_t) = 0;
   virtual void kernelInfo(int which, long long *out) = 0;
@@ -560,6 +562,21 @@ public:
                                                                      count, io);
     launched("taskKernel");
     record(s);
+  }
+  void taskLog(const DuckTask &t, const unsigned char *failed, const void *diag,
+               const void *commands, const void *filtered, double speed, void *out,
+               hipStream_t s) override {
+    DeviceGuard guard(device);
+    const int rows = blocks64(count);
+    wait(s);
+    taskLogKernel<R, B, J, CG, CS><<<rows, 64, 0, s>>>(
+        t, dStates, blobBytes, count, failed, static_cast<const R *>(diag),
+        static_cast<const R *>(commands), static_cast<const R *>(filtered),
+        R(std::max(speed, 1e-8)), static_cast<R *>(out));
+    launched("taskLogKernel");
+    record(s);
+    taskLogReduceKernel<R><<<1, 64, 0, s>>>(rows, count, static_cast<R *>(out));
+    launched("taskLogReduceKernel");
   }
   void servoSubstep(const DuckServo &p, const DuckServoSubstep &io, hipStream_t s) override {
     DeviceGuard guard(device);
@@ -1126,6 +1143,20 @@ int duck_task_reset_inputs(void *handle, const DuckTask *task, const unsigned ch
     require(std::isfinite(command_speed), "task reset inputs: command speed not finite");
     b->taskResetInputs(*task, reset_mask, joint_draws, root_draws, selected, direction,
                        command_speed, commands, q, roots, commands_out, st(hip_stream));
+  });
+}
+int duck_task_log(void *handle, const DuckTask *task, const unsigned char *failed,
+                  const void *diag, const void *commands, const void *filtered,
+                  double command_speed, void *out, void *hip_stream) {
+  return guarded([&] {
+    auto *b = as(handle);
+    checkTask(b, task);
+    require(failed && diag && out, "task log: null buffer");
+    const bool locomotion = task->kind == DUCK_TASK_LOCOMOTION;
+    require(!locomotion || commands, "task log: commands required");
+    require(!(locomotion && task->velocity_filter) || filtered,
+            "task log: filtered velocity required");
+    b->taskLog(*task, failed, diag, commands, filtered, command_speed, out, st(hip_stream));
   });
 }
 int duck_task_observe(void *handle, const DuckTask *task, const unsigned char *reset_mask,

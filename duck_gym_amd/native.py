@@ -62,6 +62,7 @@ def library():
             "duck_task_targets": (ip, [vp, ctypes.POINTER(DuckTask)] + [vp] * 7),
             "duck_task_step": (ip, [vp, ctypes.POINTER(DuckTask)] + [vp] * 13),
             "duck_task_observe": (ip, [vp, ctypes.POINTER(DuckTask)] + [vp] * 9),
+            "duck_task_log": (ip, [vp, ctypes.POINTER(DuckTask), vp, vp, vp, vp, dbl, vp, vp]),
             "duck_task_reset_inputs": (ip, [vp, ctypes.POINTER(DuckTask), vp, vp, vp, vp, ip, dbl,
                                             vp, vp, vp, vp, vp]),
             "duck_servo": (ip, [vp, ctypes.POINTER(DuckServo), vp, vp, ip] + [vp] * 7),
@@ -84,7 +85,7 @@ EXPORTED = (
     "duck_generalized_loads", "duck_reference", "duck_reference_noalloc", "duck_state_layout",
     "duck_export_state",
     "duck_import_state", "duck_last_error", "duck_task_obs_dim", "duck_task_targets",
-    "duck_task_step", "duck_task_observe", "duck_task_reset_inputs", "duck_servo",
+    "duck_task_step", "duck_task_observe", "duck_task_log", "duck_task_reset_inputs", "duck_servo",
     "duck_servo_substep",
     "duck_sequential_step",
 )
@@ -126,6 +127,7 @@ class DuckServoSubstep(ctypes.Structure):
 
 
 TASK_STANDING, TASK_LOCOMOTION, TASK_ROLLOUT = 0, 1, 2
+TASK_LOGS = 7
 
 
 class DuckTask(ctypes.Structure):
@@ -486,6 +488,23 @@ class CudaBatch:
             code = library().duck_task_step(self._h, ctypes.byref(task), *args, self._stream())
         if code:
             _raise(code, "task_step")
+
+    def task_log(self, task, failed, diag, commands, filtered, command_speed):
+        """The scalars TensorEnv.step logs (duck_task_log): a tensor of failed
+        fraction, maximum hinge error, maximum penetration and, for the
+        locomotion task, the means of |v - command|, of the velocity along the
+        command, of the reward velocity's error and of |yaw|."""
+        E = self.num_envs
+        args = [self._check(failed, [E], torch.bool), self._check(diag, [E, 6]),
+                self._ptr(commands, [E, 2]), self._ptr(filtered, [E, 2])]
+        out = self._empty(1 + (E + 63) // 64, TASK_LOGS)
+        with torch.cuda.device(self.device):
+            code = library().duck_task_log(self._h, ctypes.byref(task), *args,
+                                           float(command_speed), ctypes.c_void_p(out.data_ptr()),
+                                           self._stream())
+        if code:
+            _raise(code, "task_log")
+        return out[0]
 
     def task_observe(self, task, reset_mask, actions, commands, episode, filtered, returns,
                      forces, obs):

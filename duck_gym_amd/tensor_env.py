@@ -8,6 +8,7 @@ bookkeeping (tensor_env.py:178-219, 221-391).  Here the same step is
   task_targets  clamp(actions) and servo targets              (1 launch)
   step          the AVBD physics, `substeps` steps per launch (1 launch)
   task_step     failure, reward, counters, observation, diag  (1 launch)
+  task_log      the scalars the step logs                     (2 launches)
   reset         the torch random draws of the reference, the masked state
                 reset and a task_observe launch for the reset bookkeeping and
                 the post-reset observation
@@ -302,7 +303,9 @@ class TensorEnv:
         self.native.task_step(self.spec, a, self.actions, self._commands,
                               self.episode_length_buf, self._filtered, self.returns, obs, reward,
                               failed, timeout, done, diag)
-        peaks = diag[:, :2].amax(0)  # the two maxima in one reduction
+        # the logged scalars as views of one tensor (duck_task_log)
+        log = self.native.task_log(self.spec, failed, diag, self._commands, self._filtered,
+                                   self.command_speed).unbind()
         info = {
             "observations": {},
             "time_outs": timeout,
@@ -312,22 +315,17 @@ class TensorEnv:
             "terminal_observation": obs,
             "terminal_mask": done,
             "log": {
-                "physics/failed_fraction": failed.mean(dtype=torch.float32),
-                "physics/max_joint_error_m": peaks[0],
-                "physics/max_penetration_m": peaks[1],
+                "physics/failed_fraction": log[0].float(),
+                "physics/max_joint_error_m": log[1],
+                "physics/max_penetration_m": log[2],
             },
         }
         if self.task == "locomotion":
-            b, _, _, _, _, _, yaw = self.state()
-            velocity = self.filtered_velocity if self.velocity_filter_seconds > 0 \
-                else b[:, 1, 7:9]
-            error = (velocity - self.commands).square().sum(-1)
-            direction = self.commands / max(self.command_speed, 1e-8)
             info["log"].update({
-                "tracking/instant_error_mps": (b[:, 1, 7:9] - self.commands).norm(dim=-1).mean(),
-                "tracking/command_direction_mps": (b[:, 1, 7:9] * direction).sum(-1).mean(),
-                "tracking/reward_velocity_error_mps": error.sqrt().mean(),
-                "tracking/absolute_yaw_rad": torch.atan2(yaw[:, 1], yaw[:, 0]).abs().mean(),
+                "tracking/instant_error_mps": log[3],
+                "tracking/command_direction_mps": log[4],
+                "tracking/reward_velocity_error_mps": log[5],
+                "tracking/absolute_yaw_rad": log[6],
             })
         if self.auto_reset:
             self.reset(done)

@@ -239,6 +239,19 @@ int duck_task_observe(void *handle, const DuckTask *task, const unsigned char *r
                       void *actions, const void *commands, long long *episode, void *filtered,
                       float *returns, void *forces, float *obs, void *hip_stream);
 
+/* The scalars TensorEnv.step logs (tensor_env.py:367-391), in batch dtype,
+ * from duck_task_step's `failed` [E] and `diag` [E,6] and, for the locomotion
+ * task, the state, `commands` [E,2] and (with velocity_filter) `filtered`
+ * [E,2]: out[0..6] = failed fraction, maximum hinge error, maximum
+ * penetration, and the means of |v - command|, of v . command / max(speed,
+ * 1e-8), of the reward velocity's error and of |yaw| (zeros for the other
+ * tasks).  `out` holds (1 + ceil(E / 64)) rows of 7; the rows after the first
+ * are scratch. */
+#define DUCK_TASK_LOGS 7
+int duck_task_log(void *handle, const DuckTask *task, const unsigned char *failed,
+                  const void *diag, const void *commands, const void *filtered,
+                  double command_speed, void *out, void *hip_stream);
+
 /* ---- BAM servo substep (python/duck_gym/bam_env.py:307-326) ----
  * Parameters of the XL330/m6 actuator equations (python/duck_gym/actuator.py:
  * 16-77; names as in the BAM parameter dictionary and the official config). */

@@ -237,3 +237,37 @@ def test_env_counts_around_a_wave(model_dir, task, kind, envs):
     gen = torch.Generator(device=DEV).manual_seed(envs)
     for _ in range(2):
         _check_step(env, kind, torch.rand(envs, 14, generator=gen, device=DEV) * 2.4 - 1.2, 1e-5)
+
+
+@pytest.mark.parametrize("envs", [1, 63, 64, 65, 4200])
+@pytest.mark.parametrize("task,seconds", [("standing", 0.0), ("locomotion", 0.0), ("locomotion", 0.1)])
+def test_logged_scalars(model_dir, task, seconds, envs):
+    """The log launches against the torch expressions of tensor_env.py:367-391
+    on the same state, in float64 (sums of up to 4200 terms in another order:
+    4200 roundings of terms of the sum's own size at most).  A NaN reaches
+    the maximum, as torch.amax hands it on."""
+    env = TensorEnv(model_dir, envs, ITER, DT, 1, seed=5, task=task, auto_reset=False, fp64=True,
+                    velocity_filter_seconds=seconds)
+    actions = torch.rand(envs, 14, device=DEV, dtype=torch.float64) - 0.5
+    for _ in range(3):
+        info = env.step(actions)[3]
+    log, diag = info["log"], info["diagnostics"]
+    close = lambda a, b: torch.testing.assert_close(a, b, rtol=4200 * 2.0 ** -52, atol=0)  # noqa: E731
+    assert log["physics/failed_fraction"].dtype == torch.float32
+    close(log["physics/failed_fraction"].double(), info["failed"].mean(dtype=torch.float32).double())
+    assert log["physics/max_joint_error_m"] == diag[:, 0].max()
+    assert log["physics/max_penetration_m"] == diag[:, 1].max()
+    if task == "locomotion":
+        b, *_, yaw = env.state()
+        v = b[:, 1, 7:9]
+        error = ((env.filtered_velocity if seconds else v) - env.commands).square().sum(-1)
+        along = env.commands / max(env.command_speed, 1e-8)
+        close(log["tracking/instant_error_mps"], (v - env.commands).norm(dim=-1).mean())
+        torch.testing.assert_close(log["tracking/command_direction_mps"], (v * along).sum(-1).mean(),
+                                   rtol=0, atol=4200 * 2.0 ** -52)  # terms of either sign, below 1
+        close(log["tracking/reward_velocity_error_mps"], error.sqrt().mean())
+        close(log["tracking/absolute_yaw_rad"], torch.atan2(yaw[:, 1], yaw[:, 0]).abs().mean())
+    diag[envs // 2, 1] = float("nan")
+    again = env.native.task_log(env.spec, info["failed"], diag, env._commands, env._filtered,
+                                env.command_speed)
+    assert again[1] == diag[:, 0].max() and bool(again[2].isnan())
