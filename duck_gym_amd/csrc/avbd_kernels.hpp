@@ -18,6 +18,11 @@ template <int N> __device__ __forceinline__ double rowRor(double v) {
   return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
+// The value, opaque to the compiler from here on: what is computed from it
+// (LDS addresses, mostly) is computed anew rather than held in registers
+// across the loop that comes back here.
+__device__ __forceinline__ void keep(int &v) { asm volatile("" : "+v"(v)); }
+
 // Maximum over the L lanes of an environment, on every one of them.  For
 // L == 16 (one DPP row) four row rotations replace the LDS-crossbar shuffles.
 // c ? a : b on copies: a conditional on two lvalues of a struct type selects
@@ -186,7 +191,7 @@ __device__ __forceinline__ void dmaChunks(const unsigned char *src, __attribute_
 // kWarmContacts ground contacts as one range and, with `bodies`, the
 // reset-only group.  Environment g of the wave is e0 + g.
 constexpr int kWarmContacts = 8;
-template <class S, int G, class Env>
+template <class S, int G, bool Prefix = false, class Env>
 __device__ void loadHot(Env *envs, unsigned char *states, long long blobBytes, int e0, int count, int t,
                         bool bodies) {
   constexpr int CGcap = int(sizeof(S::gc) / sizeof(S::gc[0]));
@@ -203,7 +208,7 @@ __device__ void loadHot(Env *envs, unsigned char *states, long long blobBytes, i
     const unsigned char *blob = states + blobBytes * (e0 + g);
     auto *lds = (__attribute__((address_space(3))) unsigned char *)(&envs[g].s);
     dmaChunks<(warm - hot) / 16>(blob + hot, lds + hot, t);
-    if (bodies)
+    if (!Prefix && bodies) // (a record that holds the blob's prefix only has no such group)
       dmaChunks<(end - reset) / 16>(blob + reset, lds + reset, t);
   }
 }
@@ -691,24 +696,51 @@ __global__ void framesKernel(const DeviceModel<R> *model, Frames<R, B, J> *out) 
   stageFrames<R, B, J>(*out, *model, threadIdx.x, blockDim.x);
 }
 
-template <class R, int B, int J, int CG, int CS, int L, int PL, bool Servo, bool Pairs>
-__device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R> &sv) {
-  constexpr int G = 64 / L;
+//
+// `block` is the wave's number: it advances environments block * G + g.
+// Dense: the step of target controls of a model without body pairs with two
+// waves per SIMD -- kDenseWaves waves per workgroup, each on its own (they
+// share the Frames copy and meet once, after it has landed), on records that
+// hold what no other field gives and the first kDenseContacts ground contacts
+// (DenseEnv); further contacts stay in the blob.  The operations are the full
+// step's in its order: bitwise the same states.
+template <class R, int B, int J, int CG, int CS, int L, int PL, bool Servo, bool Pairs, bool Dense = false>
+__device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R> &sv, int block) {
+  static_assert(!Dense || (!Servo && !Pairs && sizeof(R) == sizeof(float) && L == 16 && B <= L && J <= L &&
+                           kDenseContacts <= CG),
+                "the dense step is the MicroDuck-sized float step");
+  constexpr int G = 64 / L, W = Dense ? kDenseWaves : 1;
+  constexpr int CL = Dense ? kDenseContacts : CG; // contacts a record holds
+  static_assert(kDenseContacts >= kWarmContacts, "a record holds the first copied range");
+  // The lanes of a wave meet (LDS operations of one wave complete in order; a
+  // workgroup of one wave has the barrier elided).
+  auto meet = [] {
+    if constexpr (Dense) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+      __syncthreads();
+    }
+  };
   // Lanes per body-pair query, pairs per round and rounds (pairs <= CS).
   constexpr int MQ = sizeof(R) == sizeof(float) && 2 * CS <= L ? 2 : 1;
   constexpr int PR = L / MQ;
   constexpr int PPL = (CS + PR - 1) / PR;
   constexpr int SPL = (B + L - 1) / L;  // shapes per lane (shapes <= B)
-  using Env = EnvLds<R, B, J, CG, CS, L>;
+  using Step = Stepper<R, B, J, CG, CS, L, PL, Pairs, Dense>;
+  using Env = typename Step::Env;
   using State = EnvState<R, B, J, CG, CS>;
   __shared__ Frames<R, B, J> F;
-  __shared__ Env envs[G];
+  __shared__ Env envsOf[W * G];
+  __shared__ R channels[Dense ? 3 : 1][J];
 
   const DeviceModel<R> &M = *static_cast<const DeviceModel<R> *>(args.model);
   const V3<R> *points = static_cast<const V3<R> *>(args.points);
-  const int t = threadIdx.x, lane = t % L, g = t / L;
-  const int e = xcdBlock(blockIdx.x, gridDim.x) * G + g;
+  const int t = Dense ? int(threadIdx.x % 64) : int(threadIdx.x), wave = Dense ? int(threadIdx.x / 64) : 0;
+  const int lane = t % L, g = t / L;
+  const int e = block * G + g;
   const bool valid = e < args.count;
+  Env *envs = envsOf + wave * G;
   Env &E = envs[g];
   // (a model without body pairs: none of their code is compiled)
   const int nb = args.nb, nj = args.nj, ns = args.ns, np = Pairs ? args.np : 0;
@@ -750,29 +782,58 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     auto *dst = (__attribute__((address_space(3))) uint4 *)(&F);
 #pragma unroll
     for (int k = 0; k < (FC + 63) / 64; ++k)
-      if (t + 64 * k < FC)
+      if (t + 64 * k < FC && (W == 1 || k % W == wave))
         __builtin_amdgcn_global_load_lds(src + t + 64 * k, dst + 64 * k, 16, 0, 0);
   }
 
   State *gs = valid ? &blobAt<State>(args.states, args.blobBytes, e) : nullptr;
+  if constexpr (Dense) {
+    using Record = DenseState<R, B, J, CL>;
+    static_assert(offsetof(Record, diag) == offsetof(State, diag) && offsetof(Record, x) == offsetof(State, x) &&
+                      offsetof(Record, failed) == offsetof(State, failed) &&
+                      offsetof(Record, gc) == offsetof(State, gc),
+                  "a dense record starts as the blob does");
+  }
   static_assert(L >= 4, "blob copies give each of the first three lanes an end word");
   static_assert(CS <= B, "the staged pair table holds B pairs");
-  loadHot<State, G>(envs, args.states, args.blobBytes, e - g, args.count, t, args.bodies != 0);
-  if (valid) {
-    loadEnv<State>(E.s, gs, lane, L, args.motorMode == kHeldControls, args.motorMode == kMotorControls);
-    if (!args.bodies) {
-      // the model's masses, inertia and shape friction, as reset writes them
-      for (int b = lane; b < B; b += L) {
-        E.s.mass[b] = b < nb ? M.mass[b] : R(0);
+  loadHot<State, G, Dense>(envs, args.states, args.blobBytes, e - g, args.count, t, args.bodies != 0);
+  if constexpr (Dense) {
+    if (wave == 0 && t < J) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-          E.s.inertia[k][b] = b < nb ? M.inertia[k][b] : R(0);
-      }
+      for (int k = 0; k < 3; ++k)
+        channels[k][t] = t < nj ? defs[0][k] : R(0);
+    }
+    if (valid) {
+      constexpr int gcWords = int(sizeof(GroundContact<R>) / 4), header = int(headerBytes<State>() / 4);
+      const int live = gs->ngc < 0 ? 0 : (gs->ngc < CL ? gs->ngc : CL);
+      copyWords<4>(reinterpret_cast<unsigned *>(&E.s), reinterpret_cast<const unsigned *>(gs),
+                   header + kWarmContacts * gcWords, header + live * gcWords, lane, L);
+      for (int i = int(diagBegin<State>() / 32 * 8) + lane; i < int(diagBegin<State>() / 4); i += L)
+        reinterpret_cast<unsigned *>(&E.s)[i] = 0; // as loadEnv: the lead words of the first sector written
+      if (lane < B)
+        E.s.mass[lane] = args.bodies ? gs->mass[lane] : (lane < nb ? M.mass[lane] : R(0));
       if (lane == 0)
-        E.s.friction = R(-1);
+        E.s.friction = args.bodies ? gs->friction : R(-1);
     }
   }
-  // every load of this wave, the Frames image's included, has landed
+  if constexpr (!Dense) {
+    if (valid) {
+      loadEnv<State>(E.s, gs, lane, L, args.motorMode == kHeldControls, args.motorMode == kMotorControls);
+      if (!args.bodies) {
+        // the model's masses, inertia and shape friction, as reset writes them
+        for (int b = lane; b < B; b += L) {
+          E.s.mass[b] = b < nb ? M.mass[b] : R(0);
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            E.s.inertia[k][b] = b < nb ? M.inertia[k][b] : R(0);
+        }
+        if (lane == 0)
+          E.s.friction = R(-1);
+      }
+    }
+  }
+  // every load of this wave, the Frames image's included, has landed (and, of
+  // a dense workgroup, its other waves': they share the image)
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   // The staged default schedule applies to this env while no body-body
@@ -804,7 +865,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       bad = 1;
   }
   bad = groupOr<L>(bad);
-  __syncthreads();
+  meet();
   bool active = false;
   // What the blob's drive parameters and colouring hold before this launch
   // (read before any lane rewrites the stamps).
@@ -817,7 +878,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       // State::advance (kernel.cuh:421-443): the controls in the state as
       // they stand
       active = !E.s.failed;
-    } else if (args.motorMode == kMotorControls) {
+    } else if (!Dense && args.motorMode == kMotorControls) {
+      if constexpr (!Dense) {
       // setMotor applies the channels even when they are invalid (slots
       // past the last hinge hold zeros, as the state was created).
 #pragma unroll
@@ -842,6 +904,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       driveWrite = driveIn == kDriveMotor ? kWriteMotorDrive : kWriteDrive;
       writeFrom = int(forceBegin<State>() / 32 * 8);
       active = !E.s.failed && !bad;
+      }
     } else if (!E.s.failed && !bad) {
       const R kp = R(args.kp), limit = R(args.limit);
       const bool same = driveIn == kDriveTarget && sameBits(E.s.driveKp, kp) && sameBits(E.s.driveLimit, limit);
@@ -853,11 +916,13 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         // slots past the last hinge hold zeros, as the state was created
         const bool in = j < nj;
         E.s.target[j] = in ? ctl[r][0] : R(0);
-        E.s.kp[j] = in ? kp : R(0);
-        E.s.maxTorque[j] = in ? limit : R(0);
-        E.s.torque[j] = in ? defs[r][0] : R(0);
-        E.s.frictionloss[j] = in ? defs[r][1] : R(0);
-        E.s.damping[j] = in ? defs[r][2] : R(0);
+        if constexpr (!Dense) {
+          E.s.kp[j] = in ? kp : R(0);
+          E.s.maxTorque[j] = in ? limit : R(0);
+          E.s.torque[j] = in ? defs[r][0] : R(0);
+          E.s.frictionloss[j] = in ? defs[r][1] : R(0);
+          E.s.damping[j] = in ? defs[r][2] : R(0);
+        }
       }
       if (lane < 3)
         E.s.force[lane] = fin;
@@ -889,12 +954,22 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       E.s.diag[k] = k == kConverged ? R(1) : R(0);
     }
   }
-  __syncthreads();
+  meet();
 
-  Stepper<R, B, J, CG, CS, L, PL, Pairs> stp{M, points, F, E, lane};
+  Step stp{M, points, F, E, lane, {}};
+  if constexpr (Dense)
+    stp.common = {R(args.kp), R(args.limit), channels, gs ? gs->gc : nullptr, __any(valid && E.s.ngc > CL) != 0};
+  // The lanes that share contacts in the blobs meet behind a fence.
+  auto meetFar = [&] {
+    if constexpr (Dense) {
+      if (stp.common.far)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    }
+    meet();
+  };
   // Block-solve lanes: with P == 2, lanes l and l ^ 8 (same 16-lane DPP row)
   // share a body; `slot` numbers the bodies a colour pass runs at once.
-  constexpr int P = Stepper<R, B, J, CG, CS, L, PL, Pairs>::P;
+  constexpr int P = Step::P;
   static_assert(P == 1 || L % (8 * P) == 0, "split block solves need 8 P-lane groups");
   const int part = (lane >> 3) & (P - 1);
   const int slot = P == 1 ? lane : (lane & 7) + 8 * (lane / (8 * P));
@@ -912,6 +987,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       int src;
     };
     PairGeom pg[PPL];
+    if constexpr (!Dense)
 #pragma unroll
     for (int r = 0; r < PPL; ++r) {
       // the lanes of a query compute the same values and branch alike; the
@@ -1136,7 +1212,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         int ids[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          ids[j] = E.s.gc[i0 + j < ngc ? i0 + j : 0].id;
+          ids[j] = stp.groundId(i0 + j < ngc ? i0 + j : 0);
 #pragma unroll
         for (int j = 3; j >= 0; --j) {
           const int masked = i0 + j < ngc ? ids[j] & kGcShapeFeature : -2;
@@ -1151,7 +1227,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
           picks[r][p] |= src[p] << 20;
         // the source's multipliers, penalties and stick anchor, read while
         // the previous list is still in LDS (compaction overwrites it)
-        const GroundContact<R> &old = E.s.gc[p < n && src[p] > 0 ? src[p] - 1 : 0];
+        const auto &old = stp.template ground<Dense>(p < n && src[p] > 0 ? src[p] - 1 : 0);
         WarmGround &wm = warm[r][p];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -1164,7 +1240,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         wm.stick = gcStick(old.id);
       }
     }
-    __syncthreads();
+    meetFar();
     // ---------------- compaction + warm start ----------------------------
     if (active) {
       int total = 0;
@@ -1220,12 +1296,12 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
             c.lambda[d] = lam[d] * ag;
             c.penalty[d] = clampv(pen[d] * gamma, R(1000), R(1e9));
           }
-          E.s.gc[offset + p] = c;
-          clearContactPadding(E.s.gc[offset + p]);
+          stp.putGround(offset + p, c);
         }
       }
       if (lane == 0)
         E.s.ngc = total > CG ? CG : total;
+      if constexpr (!Dense)
 #pragma unroll
       for (int r = 0; r < PPL; ++r) {
         const int pi = lane / MQ + r * PR;
@@ -1266,16 +1342,22 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         clearContactPadding(E.s.sc[slot]);
       }
     }
-    __syncthreads();
+    if constexpr (Dense) {
+      meet();
+      stp.common.far = stp.common.far || __any(active && E.s.ngc > CL);
+    }
+    meetFar();
     // ---------------- colours (kernel.cuh:596-598, 717-720) -------------
     int pairHits = 0;
-    for (int pi = 0; pi < np; ++pi)
-      pairHits += E.pairHit[pi];
+    if constexpr (!Dense)
+      for (int pi = 0; pi < np; ++pi)
+        pairHits += E.pairHit[pi];
     const bool fresh = active && !(pairHits == 0 && defaultSchedule);
     if (active) {
       for (int b = lane; b < B; b += L) {
         // slots past the last body hold zeros, as the state was created
-        E.s.colors[b] = b < nb ? M.colors[b] : 0;
+        if constexpr (!Dense)
+          E.s.colors[b] = b < nb ? M.colors[b] : 0;
         if (!fresh && b < nb)
           E.order[b] = F.order[b];
       }
@@ -1288,21 +1370,22 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         E.s.colorCount = 2;
       }
     }
-    __syncthreads();
+    meet();
     if (fresh && lane == 0) {
       // each body contact between bodies of one colour gives its second
       // body a new colour, in list order (later contacts see the change)
       const int nsc = pairHits < CS ? pairHits : CS;
       E.s.nsc = nsc;
       int cc = 2;
-      for (int i = 0; i < nsc; ++i) {
-        int a = scBody(E.s.sc[i].id), b = scOther(E.s.sc[i].id);
-        if (E.s.mass[a] > 0 && E.s.mass[b] > 0 && E.s.colors[a] == E.s.colors[b])
-          E.s.colors[b] = cc++;
-      }
+      if constexpr (!Dense)
+        for (int i = 0; i < nsc; ++i) {
+          int a = scBody(E.s.sc[i].id), b = scOther(E.s.sc[i].id);
+          if (E.s.mass[a] > 0 && E.s.mass[b] > 0 && E.s.colors[a] == E.s.colors[b])
+            E.s.colors[b] = cc++;
+        }
       E.s.colorCount = cc;
     }
-    __syncthreads();
+    meet();
     // The fresh schedule: the dynamic bodies of each colour in index order,
     // placed by ballots over the environment's lanes (body b = lane + r L).
     const int freshColours = __builtin_amdgcn_readfirstlane(waveMaxInt(fresh ? E.s.colorCount : 0));
@@ -1313,7 +1396,10 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
 #pragma unroll
       for (int r = 0; r < BR; ++r) {
         const int b = lane + r * L;
-        col[r] = fresh && b < nb && E.s.mass[b] > 0 ? E.s.colors[b] : -1;
+        if constexpr (Dense)
+          col[r] = fresh && b < nb && E.s.mass[b] > 0 ? M.colors[b] : -1;
+        else
+          col[r] = fresh && b < nb && E.s.mass[b] > 0 ? E.s.colors[b] : -1;
       }
       int start = 0;
       for (int c = 0; c <= freshColours; ++c) {
@@ -1331,7 +1417,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         }
       }
     }
-    __syncthreads();
+    meet();
     if (active && E.s.failed)
       active = false; // detection failure ends this env's launch
     // ---------------- warm start, predictor, contact masks ---------------
@@ -1339,7 +1425,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       for (int ji = lane; ji < nj; ji += L) {
         auto je = stp.evalJoint(ji);
 #pragma unroll
-        for (int k = 0; k < 7; ++k)
+        for (int k = 0; k < (Dense ? 5 : 7); ++k)
           E.c0[k][ji] = je.C[k];
         E.angle0[ji] = je.angle;
         E.s.lambdaF[ji] *= ag;
@@ -1362,39 +1448,44 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
 #pragma unroll
         for (int k = 0; k < GW; ++k)
           E.gmask[k][b] = 0;
-        E.smask[b] = 0;
+        if constexpr (!Dense)
+          E.smask[b] = 0;
       }
     }
-    __syncthreads(); // joint warm start reads the poses the predictor overwrites
+    meet(); // joint warm start reads the poses the predictor overwrites
     if (active) {
       for (int i = lane; i < E.s.ngc; i += L)
-        atomicOr(reinterpret_cast<unsigned long long *>(&E.gmask[i >> 6][gcBody(E.s.gc[i].id)]),
+        atomicOr(reinterpret_cast<unsigned long long *>(&E.gmask[i >> 6][gcBody(stp.groundId(i))]),
                  1ull << (i & 63));
-      for (int i = lane; i < E.s.nsc; i += L) {
-        const int id = E.s.sc[i].id;
-        atomicOr(&E.smask[scBody(id)], 1u << i);
-        atomicOr(&E.smask[scOther(id)], 1u << i);
-      }
+      if constexpr (!Dense)
+        for (int i = lane; i < E.s.nsc; i += L) {
+          const int id = E.s.sc[i].id;
+          atomicOr(&E.smask[scBody(id)], 1u << i);
+          atomicOr(&E.smask[scOther(id)], 1u << i);
+        }
       for (int b = lane; b < nb; b += L) {
         V3<R> x = stp.X(b);
         Q4<R> q = stp.Q(b);
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          E.x0[k][b] = comp(x, k);
-        E.q0[0][b] = q.w;
-        E.q0[1][b] = q.x;
-        E.q0[2][b] = q.y;
-        E.q0[3][b] = q.z;
+        V3<R> I;
+        if constexpr (Dense)
+          I = args.bodies ? V3<R>{gs->inertia[0][b], gs->inertia[1][b], gs->inertia[2][b]}
+                          : V3<R>{M.inertia[0][b], M.inertia[1][b], M.inertia[2][b]};
+        else
+          I = stp.Inertia(b);
+        if constexpr (!Dense)
+          stp.setStart(b, x, q);
         {
           R iw[6];
-          inertiaWorld(q, stp.Inertia(b), iw);
+          inertiaWorld(q, I, iw);
           for (int k = 0; k < 6; ++k)
             E.Iw[k][b] = iw[k];
         }
         const R mass = E.s.mass[b];
         if (mass == 0)
           continue;
-        V3<R> v = stp.Vel(b), w = stp.Omega(b), I = stp.Inertia(b);
+        V3<R> v = stp.Vel(b), w = stp.Omega(b);
+        if constexpr (Dense)
+          stp.setStart(b, x, q); // over the velocities just read
         V3<R> xp = faxpy(h * h, V3<R>{M.gravity[0], M.gravity[1], M.gravity[2]} + divide(stp.force(b), mass),
                          faxpy(h, v, x));
         V3<R> spin = -cross(w, stp.inertiaApply(q, I, w, false));
@@ -1412,7 +1503,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       }
     }
     int colours = waveMaxInt(active ? E.s.colorCount : 0);
-    __syncthreads();
+    meet();
     // When each of the first two colours fits in one pass of the block-solve
     // slots, every lane's body for them is fixed for the whole step.
     bool twoColourSlots = false;
@@ -1515,7 +1606,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       }
     }
     // The lane's assembly plans for its bodies of the first two colours.
-    typename Stepper<R, B, J, CG, CS, L, PL, Pairs>::SlotPlan plans[2] = {{0, 0}, {0, 0}};
+    typename Step::SlotPlan plans[2] = {{0, 0}, {0, 0}};
     if constexpr (sizeof(R) == sizeof(float)) {
 #pragma unroll
       for (int c = 0; c < 2; ++c)
@@ -1523,7 +1614,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
           plans[c] = stp.plan(mine[c], partOf[c], partsOf[c]);
       plans[1].w0 |= stageLane ? 1 << 28 : 0;
     }
-    E.early = early ? 1 : 0;
+    if constexpr (Pairs)
+      E.early = early ? 1 : 0;
     // Which hinge's dual update a lane makes first.  A hinge's dual update
     // and the next iteration's first-colour block solve of its colour-0 body
     // evaluate it at the same poses (nothing moves in between), so when every
@@ -1556,8 +1648,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     }
     // The ends of that hinge and the owner of the lane's first ground
     // contact (the list is fixed until the next detection).
-    const int ends0 = dualJoint >= 0 ? F.a[dualJoint] | F.b[dualJoint] << 8 : F.a[0] | F.b[0] << 8;
-    typename Stepper<R, B, J, CG, CS, L, PL, Pairs>::JointEval lastEval{};
+    int ends0 = dualJoint >= 0 ? F.a[dualJoint] | F.b[dualJoint] << 8 : F.a[0] | F.b[0] << 8;
+    typename Step::JointEval lastEval{};
     int owner0 = 0;
     if (active && lane < E.s.ngc) {
       const int id = E.s.gc[lane].id;
@@ -1583,6 +1675,14 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         break;
       R maxUpdate = 0;
       for (int c = 0; c < colours; ++c) {
+        if constexpr (Dense) {
+          keep(mine[0]);
+          keep(mine[1]);
+          keep(plans[0].w0);
+          keep(plans[0].w1);
+          keep(plans[1].w0);
+          keep(plans[1].w1);
+        }
         const bool quadPass = c == 0 ? quadPass0 : (c == 1 ? quadPass1 : false);
         if (work && c < E.s.colorCount) {
           if (c < 2 && twoColourSlots) {
@@ -1600,15 +1700,23 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
             // (an early-assembled third colour is its one body: slot 0)
             for (int k = E.colorStart[c] + slot; k < E.colorStart[c + 1]; k += L / P) {
               const int bi = E.order[k];
+              bool finish = false;
+              if constexpr (Pairs)
+                finish = c == 2 && E.early != 0;
               maxUpdate = mx(maxUpdate, stp.updateBody(bi, true, part, P, false, stp.plan(bi, part, P),
-                                                       nullptr, c == 2 && E.early != 0));
+                                                       nullptr, finish));
             }
           }
         }
-        __syncthreads();
+        meet();
       }
       maxUpdate = groupMax<L>(maxUpdate);
       R error = 0;
+      if constexpr (Dense) {
+        keep(dualJoint);
+        keep(ends0);
+        keep(owner0);
+      }
       if (work) {
         // The lane's first hinge and first ground contact as one straight-
         // line block (stores at its end), then any further ones; the error
@@ -1619,7 +1727,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         R errC0 = 0;
         dualRan = true;
         dJoint = dAxis = dDepth = 0;
-        auto foldJoint = [&](const typename Stepper<R, B, J, CG, CS, L, PL, Pairs>::JointDual &jd) {
+        auto foldJoint = [&](const typename Step::JointDual &jd) {
 #pragma unroll
           for (int k = 0; k < 3; ++k)
             dJoint = mx(dJoint, mabs(jd.C[k]));
@@ -1627,7 +1735,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
           for (int k = 3; k < 5; ++k)
             dAxis = mx(dAxis, mabs(jd.C[k]));
         };
-        static_assert(L <= CG, "a lane's first contact slot exists");
+        static_assert(L <= CL, "a lane's first contact slot exists");
         // a lane without a hinge evaluates an existing slot and stores nothing
         const bool hasJoint = dualJoint >= 0;
         // New force, penalties and stick flag of body contact i (kernel.cuh:
@@ -1635,24 +1743,28 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         // error (folded by the caller).
         const int nsc = E.s.nsc;
         auto selfDual = [&](int i, bool v) __attribute__((always_inline)) {
-          SelfContact<R> &c = E.s.sc[v ? i : 0];
-          V3<R> ra, rb;
-          V3<R> C = stp.selfC(c, ra, rb);
-          const R depth = mx(R(0), -(C.z + alpha * c.c0));
-          V3<R> f = contactForce(C, c.lambda, c.penalty, c.friction);
-          R trial = fhypot(fmad(c.penalty[0], C.x, c.lambda[0]), fmad(c.penalty[1], C.y, c.lambda[1]));
-          bool stick = trial <= -c.friction * f.z && double(fhypot(C.x, C.y)) < 1e-5;
-          R fk[3] = {f.x, f.y, f.z}, Ck[3] = {C.x, C.y, C.z};
-          if (v) {
-            c.id = (c.id & 0x7fffffff) | (stick ? int(0x80000000u) : 0);
+          if constexpr (Dense) {
+            return V3<R>{0, 0, 0};
+          } else {
+            SelfContact<R> &c = E.s.sc[v ? i : 0];
+            V3<R> ra, rb;
+            V3<R> C = stp.selfC(c, ra, rb);
+            const R depth = mx(R(0), -(C.z + alpha * c.c0));
+            V3<R> f = contactForce(C, c.lambda, c.penalty, c.friction);
+            R trial = fhypot(fmad(c.penalty[0], C.x, c.lambda[0]), fmad(c.penalty[1], C.y, c.lambda[1]));
+            bool stick = trial <= -c.friction * f.z && double(fhypot(C.x, C.y)) < 1e-5;
+            R fk[3] = {f.x, f.y, f.z}, Ck[3] = {C.x, C.y, C.z};
+            if (v) {
+              c.id = (c.id & 0x7fffffff) | (stick ? int(0x80000000u) : 0);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-              c.lambda[k] = fk[k];
-              if (f.z < 0 && (k == 2 || trial <= -c.friction * f.z))
-                c.penalty[k] = mn(fmad(M.betaLinear, mabs(Ck[k]), c.penalty[k]), R(1e9));
+              for (int k = 0; k < 3; ++k) {
+                c.lambda[k] = fk[k];
+                if (f.z < 0 && (k == 2 || trial <= -c.friction * f.z))
+                  c.penalty[k] = mn(fmad(M.betaLinear, mabs(Ck[k]), c.penalty[k]), R(1e9));
+              }
             }
+            return V3<R>{depth, mx(R(0), -C.z), R(0)};
           }
-          return V3<R>{depth, mx(R(0), -C.z), R(0)};
         };
         auto j0 = stp.jointDual(hasJoint ? dualJoint : (lane < J ? lane : 0), hasJoint, error, ends0);
         const auto g0 = stp.groundDual(lane, lane < ngc, errC0, owner0);
@@ -1698,8 +1810,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
           const int i = i0 + lane;
           const bool v = i < ngc;
           const int k = v ? i : lane;
-          const int id = E.s.gc[k].id;
-          const auto gd = stp.groundDual(k, v, error, v ? gcBody(id) | gcShape(id) << 8 : owner0);
+          const int id = stp.groundId(k);
+          const auto gd = stp.template groundDual<Dense>(k, v, error, v ? gcBody(id) | gcShape(id) << 8 : owner0);
           stp.storeGroundDual(k, gd);
           dDepth = v ? mx(dDepth, gd.depth) : dDepth;
         }
@@ -1723,7 +1835,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         E.stepDiag[kConverged] = conv ? R(1) : R(0);
       }
       converged = converged || (work && conv);
-      __syncthreads();
+      meetFar();
     }
     // ---------------- velocity recovery (kernel.cuh:1064-1073) ------------
     if (active) {
@@ -1731,7 +1843,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       for (int b = lane; b < nb; b += L) {
         if (E.s.mass[b] == 0)
           continue;
-        V3<R> x = stp.X(b), x0{E.x0[0][b], E.x0[1][b], E.x0[2][b]};
+        V3<R> x = stp.X(b), x0 = stp.X0(b);
         V3<R> v = (x - x0) * invh;
         V3<R> w = flogmap(fqmul(stp.Q(b), conj(stp.Q0(b)))) * invh;
 #pragma unroll
@@ -1743,7 +1855,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
           E.s.failed = 1;
       }
     }
-    __syncthreads();
+    meet();
     if (active && E.s.failed)
       active = false;
     // ---------------- diagnostics and substep summary ---------------------
@@ -1760,14 +1872,16 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       }
       for (int i = lane; i < E.s.ngc; i += L) {
         V3<R> ra;
-        V3<R> C = stp.groundC(E.s.gc[i], ra);
-        pen = mx(pen, mx(R(0), -(C.z + alpha * E.s.gc[i].c0)));
+        const auto &c = stp.template ground<Dense>(i);
+        V3<R> C = stp.groundC(c, ra);
+        pen = mx(pen, mx(R(0), -(C.z + alpha * c.c0)));
       }
-      for (int i = lane; i < E.s.nsc; i += L) {
-        V3<R> ra, rb;
-        V3<R> C = stp.selfC(E.s.sc[i], ra, rb);
-        pen = mx(pen, mx(R(0), -(C.z + alpha * E.s.sc[i].c0)));
-      }
+      if constexpr (!Dense)
+        for (int i = lane; i < E.s.nsc; i += L) {
+          V3<R> ra, rb;
+          V3<R> C = stp.selfC(E.s.sc[i], ra, rb);
+          pen = mx(pen, mx(R(0), -(C.z + alpha * E.s.sc[i].c0)));
+        }
     }
     jointErr = groupMax<L>(jointErr);
     axisErr = groupMax<L>(axisErr);
@@ -1781,8 +1895,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       d[kConverged] = (d[kConverged] != 0 && E.stepDiag[kConverged] != 0) ? R(1) : R(0);
       d[kIterations] += E.stepDiag[kIterations];
     }
-    __syncthreads();
-    __syncthreads();
+    meet();
+    meet();
   }
   if constexpr (Servo)
     if (valid && lane == 0)
@@ -1792,12 +1906,30 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   const int plan = valid ? E.writeback : 0;
   const bool modelColours = E.s.colorCount == 2;
   const bool writeColours = ran && !(modelColours && (plan & 1));
-  __syncthreads();
+  meet();
   if (ran && lane == 0)
     E.s.modelColours = modelColours ? 1 : 0;
-  __syncthreads();
-  if (valid)
+  meet();
+  if constexpr (Dense) {
+    if (valid) {
+      constexpr int gcWords = int(sizeof(GroundContact<R>) / 4), header = int(headerBytes<State>() / 4);
+      copyWords<4>(reinterpret_cast<unsigned *>(gs), reinterpret_cast<const unsigned *>(&E.s), plan >> 8,
+                   header + (E.s.ngc < CL ? E.s.ngc : CL) * gcWords, lane, L);
+      // what the record does not hold, from its sources
+      if (((plan >> 1) & 3) != kWriteNoDrive && lane < J) {
+        const bool in = lane < nj;
+        gs->kp[lane] = in ? R(args.kp) : R(0);
+        gs->maxTorque[lane] = in ? R(args.limit) : R(0);
+        gs->torque[lane] = channels[0][lane];
+        gs->frictionloss[lane] = channels[1][lane];
+        gs->damping[lane] = channels[2][lane];
+      }
+      if (writeColours && lane < B)
+        gs->colors[lane] = lane < nb ? M.colors[lane] : 0;
+    }
+  } else if (valid) {
     storeEnv<State>(gs, E.s, lane, L, plan >> 8, (plan >> 1) & 3, writeColours);
+  }
 }
 
 // Pairs false: for a model without body pairs.  The code starts on a 32 KiB
@@ -1806,7 +1938,24 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
 template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true>
 __global__ __launch_bounds__(64) __attribute__((aligned(32768))) void advanceKernel(StepArgs args) {
   const ServoArgs<R> none{};
-  stepBody<R, B, J, CG, CS, L, PL, false, Pairs>(args, none);
+  stepBody<R, B, J, CG, CS, L, PL, false, Pairs>(args, none, xcdBlock(blockIdx.x, gridDim.x));
+}
+
+// The step of a batch with more waves than SIMDs (stepBody's Dense).  The full
+// step's wave issues VALU work in 59 % of its life and its 40 KiB of LDS and
+// 400 registers admit no second one beside it, so such a batch ran in rounds;
+// here two waves share a SIMD (20 KiB and 256 registers each) and fill each
+// other's waits: VALU issue 85 % of the time, a wave's life 47.6 k -> 66.5 k
+// quad-cycles at 32768 standing environments.  Four steps of them: 2470 ->
+// 1854 us; the landed drop of 16384: 488 -> 379 us.  What is left is the issue
+// of its 27.3 k VALU instructions, and the registers that detection spills
+// (keep() keeps addresses from being spilled across the iterations: without it
+// 2233 us).
+template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L)>
+__global__ __launch_bounds__(64 * kDenseWaves, 2) __attribute__((aligned(32768))) void denseKernel(StepArgs args) {
+  const ServoArgs<R> none{};
+  stepBody<R, B, J, CG, CS, L, PL, false, false, true>(
+      args, none, xcdBlock(blockIdx.x, gridDim.x) * kDenseWaves + int(threadIdx.x / 64));
 }
 
 // One servo substep per launch (bam_env.py:307-337 with refresh()), on a
@@ -1814,7 +1963,7 @@ __global__ __launch_bounds__(64) __attribute__((aligned(32768))) void advanceKer
 template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true>
 __global__ __launch_bounds__(64) __attribute__((aligned(32768))) void servoStepKernel(StepArgs args,
                                                                                    ServoArgs<R> servo) {
-  stepBody<R, B, J, CG, CS, L, PL, true, Pairs>(args, servo);
+  stepBody<R, B, J, CG, CS, L, PL, true, Pairs>(args, servo, xcdBlock(blockIdx.x, gridDim.x));
 }
 
 } // namespace duckhip

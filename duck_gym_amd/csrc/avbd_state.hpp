@@ -18,6 +18,7 @@
 #include "avbd_math.hpp"
 
 #include <cstdint>
+#include <type_traits>
 
 namespace duckhip {
 
@@ -226,6 +227,53 @@ struct EnvLds : EnvLdsCore<R, B, J, CG, CS> {
 };
 template <class R, int B, int J, int CG, int CS, int L>
 struct EnvLds<R, B, J, CG, CS, L, 0> : EnvLdsCore<R, B, J, CG, CS> {};
+
+// LDS record of the dense step (two waves per SIMD): a step of target controls
+// for a model without body pairs.  `s` is the blob's own prefix up to the
+// CL-th contact, so that it is loaded and written back as the blob's byte
+// range (contacts from the CL-th on stay in the blob); of the rest only the
+// masses and the friction are kept.  The drive is the launch's kp and limit
+// and the model's channels (no per-environment copies), the limit rows' c0
+// follow from angle0, and a dynamic body's x0 and q0 stand in its velocity
+// rows between the predictor, which reads the velocities last, and the
+// recovery, which writes them.
+template <class R, int B, int J, int CL> struct DenseState {
+  unsigned char lead[leadBytes<R, J>()];
+  R diag[8];
+  R target[J];
+  R force[3];
+  R x[3][B];
+  R q[4][B], v[3][B], w[3][B];
+  R lambda[7][J], penalty[7][J];
+  R lambdaF[J], penaltyF[J];
+  int failed, ngc, nsc, colorCount;
+  int drive, modelColours;
+  R driveKp, driveLimit;
+  alignas(16) GroundContact<R> gc[CL];
+  R mass[B];
+  R friction;
+};
+template <class R, int B, int J, int CL> struct DenseEnvCore {
+  DenseState<R, B, J, CL> s;
+  R q0z[B], xp[3][B], qp[4][B];
+  R Iw[6][B];
+  R c0[5][J], angle0[J], velocity0[J];
+  R stepDiag[8];
+  uint64_t gmask[1][B];
+  int order[B], colorStart[3];
+  int writeback;
+  int shapeCount[B];
+};
+template <class R, int B, int J, int CL, int L,
+          int Pad = bankPadWords<int(sizeof(DenseEnvCore<R, B, J, CL>) / 4), L>()>
+struct DenseEnv : DenseEnvCore<R, B, J, CL> {
+  int bankPad[Pad];
+};
+template <class R, int B, int J, int CL, int L>
+struct DenseEnv<R, B, J, CL, L, 0> : DenseEnvCore<R, B, J, CL> {};
+// Waves per workgroup of the dense step (they share one Frames copy) and the
+// contacts its records hold: as many as fit eight waves into a CU's 160 KiB.
+constexpr int kDenseWaves = 4, kDenseContacts = 23;
 
 // Byte offsets of the ground-contact list inside the blob (only its live
 // entries are copied), of the diagnostics, the targets, the force and group 1,

@@ -341,17 +341,33 @@ template <int N> __device__ __forceinline__ double rowRotate(double v) {
 // environment, two with 16, four with 32.
 constexpr int defaultSolveLanes(int L) { return L >= 32 ? 4 : (L >= 16 ? 2 : 1); }
 
+// What a dense step holds outside its record: the launch's gains, the model's
+// channels (torque, frictionloss, damping; staged once per workgroup), and the
+// environment's contact list in its blob, where the contacts from the
+// kDenseContacts-th on stay; `far` says that an environment of the wave has
+// some (in the list before or after a detection).
+template <class R, int J> struct DenseShare {
+  R kp, limit;
+  const R (*channels)[J];
+  GroundContact<R> *list;
+  bool far;
+};
+struct NoShare {};
+
 // Pairs: the model may have body-body contacts (without them, the rows and
-// the two-pass assembly of body contacts are left out).
-template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true>
+// the two-pass assembly of body contacts are left out).  Dense: the records
+// are the dense step's.
+template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true,
+          bool Dense = false>
 struct Stepper {
-  using Env = EnvLds<R, B, J, CG, CS, L>;
+  using Env = std::conditional_t<Dense, DenseEnv<R, B, J, kDenseContacts, L>, EnvLds<R, B, J, CG, CS, L>>;
   using Fr = Frames<R, B, J>;
   const DeviceModel<R> &M;
   const V3<R> *points;
   const Fr &F;
   Env &E;
   int lane; // 0..L-1 within the environment
+  std::conditional_t<Dense, DenseShare<R, J>, NoShare> common;
   // Lanes per block solve: one (the reference's accumulation order), or
   // with 16 lanes per environment two lanes (lane, lane ^ 8), with 32 lanes
   // four (lane ^ 8, ^ 16, ^ 24) that share each body's assembly and sum it by
@@ -394,7 +410,109 @@ struct Stepper {
   DUCK_HD V3<R> Inertia(int b) const {
     return {E.s.inertia[0][b], E.s.inertia[1][b], E.s.inertia[2][b]};
   }
-  DUCK_HD Q4<R> Q0(int b) const { return {E.q0[0][b], E.q0[1][b], E.q0[2][b], E.q0[3][b]}; }
+  // Pose at the start of the step.  Dense: in the velocity rows, for a
+  // dynamic body after the predictor.
+  DUCK_HD V3<R> X0(int b) const {
+    if constexpr (Dense)
+      return {E.s.v[0][b], E.s.v[1][b], E.s.v[2][b]};
+    else
+      return {E.x0[0][b], E.x0[1][b], E.x0[2][b]};
+  }
+  DUCK_HD Q4<R> Q0(int b) const {
+    if constexpr (Dense)
+      return {E.s.w[0][b], E.s.w[1][b], E.s.w[2][b], E.q0z[b]};
+    else
+      return {E.q0[0][b], E.q0[1][b], E.q0[2][b], E.q0[3][b]};
+  }
+  DUCK_HD void setStart(int b, V3<R> x, Q4<R> q) {
+    auto &px = [&]() -> R(&)[3][B] {
+      if constexpr (Dense)
+        return E.s.v;
+      else
+        return E.x0;
+    }();
+    px[0][b] = x.x;
+    px[1][b] = x.y;
+    px[2][b] = x.z;
+    if constexpr (Dense) {
+      E.s.w[0][b] = q.w;
+      E.s.w[1][b] = q.x;
+      E.s.w[2][b] = q.y;
+      E.q0z[b] = q.z;
+    } else {
+      E.q0[0][b] = q.w;
+      E.q0[1][b] = q.x;
+      E.q0[2][b] = q.y;
+      E.q0[3][b] = q.z;
+    }
+  }
+  // Constraint value k of hinge j at the start of the step.
+  DUCK_HD R C0(int k, int j) const {
+    if constexpr (Dense)
+      return k < 5 ? E.c0[k < 5 ? k : 0][j] : (k == 5 ? E.angle0[j] - F.lo[j] : F.hi[j] - E.angle0[j]);
+    else
+      return E.c0[k][j];
+  }
+  // Ground contact i: a reference into the record or, with Far (a dense wave
+  // with contacts in its blobs), its value from the record or the blob.
+  template <bool Far> DUCK_HD decltype(auto) ground(int i) const {
+    if constexpr (Far) {
+      GroundContact<R> c = E.s.gc[i < kDenseContacts ? i : 0];
+      if (i >= kDenseContacts)
+        c = common.list[i];
+      return c;
+    } else {
+      return static_cast<const GroundContact<R> &>(E.s.gc[i]);
+    }
+  }
+  DUCK_HD int groundId(int i) const {
+    if constexpr (Dense)
+      return i < kDenseContacts ? E.s.gc[i].id : common.list[i].id;
+    else
+      return E.s.gc[i].id;
+  }
+  __device__ void putGround(int i, const GroundContact<R> &c) {
+    if constexpr (Dense) {
+      if (i < kDenseContacts)
+        E.s.gc[i] = c;
+      else
+        common.list[i] = c;
+    } else {
+      E.s.gc[i] = c;
+      clearContactPadding(E.s.gc[i]);
+    }
+  }
+  // The drive of hinge j.
+  DUCK_HD R Kp(int j) const {
+    if constexpr (Dense)
+      return common.kp;
+    else
+      return E.s.kp[j];
+  }
+  DUCK_HD R MaxTorque(int j) const {
+    if constexpr (Dense)
+      return common.limit;
+    else
+      return E.s.maxTorque[j];
+  }
+  DUCK_HD R Torque(int j) const {
+    if constexpr (Dense)
+      return common.channels[0][j];
+    else
+      return E.s.torque[j];
+  }
+  DUCK_HD R FrictionLoss(int j) const {
+    if constexpr (Dense)
+      return common.channels[1][j];
+    else
+      return E.s.frictionloss[j];
+  }
+  DUCK_HD R Damping(int j) const {
+    if constexpr (Dense)
+      return common.channels[2][j];
+    else
+      return E.s.damping[j];
+  }
   DUCK_HD void setX(int b, V3<R> v) {
     E.s.x[0][b] = v.x;
     E.s.x[1][b] = v.y;
@@ -533,7 +651,7 @@ struct Stepper {
     R err = error;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      const R c = fmad(-alpha, E.c0[k][jg], je.C[k]);
+      const R c = fmad(-alpha, C0(k, jg), je.C[k]);
       const R pen = E.s.penalty[k][ji], lam = E.s.lambda[k][ji];
       o.lambda[k] = valid ? fmad(pen, c, lam) : lam;
       const R ramped = mn(fmad(k < 3 ? M.betaLinear : M.betaAngular, mabs(c), pen), k < 3 ? R(1e9) : R(1e7));
@@ -543,7 +661,7 @@ struct Stepper {
     const bool limited = valid & (F.limited[jg] != 0);
 #pragma unroll
     for (int k = 5; k < 7; ++k) {
-      const R c = fmad(-alpha, mn(E.c0[k][jg], R(0)), je.C[k]);
+      const R c = fmad(-alpha, mn(C0(k, jg), R(0)), je.C[k]);
       const R pen = E.s.penalty[k][ji], lam = E.s.lambda[k][ji];
       const R f = fmad(pen, c, lam);
       o.lambda[k] = limited ? mn(f, R(0)) : lam;
@@ -556,7 +674,7 @@ struct Stepper {
     for (int k = 0; k < 5; ++k)
       o.C[k] = je.C[k];
     o.angle = je.angle - E.angle0[jg];
-    o.fl = E.s.frictionloss[jg];
+    o.fl = FrictionLoss(jg);
     o.lambdaF0 = E.s.lambdaF[ji];
     o.penaltyF0 = E.s.penaltyF[ji];
     o.rough = valid & (o.fl > 0);
@@ -584,8 +702,9 @@ struct Stepper {
   };
   // `owner` is the contact's body | shape << 8 (0 when not valid), which a
   // lane may hold in a register for its first contact (fixed within a step).
+  template <bool Far = false>
   __device__ GroundDual groundDual(int i, bool valid, R &error, int owner) const {
-    const GroundContact<R> &c = E.s.gc[i];
+    const auto &c = ground<Far>(i);
     const int id = c.id;
     const int b = owner & 255, shape = owner >> 8;
     const V3<R> ra = frotate(Q(b), V3<R>{c.local[0], c.local[1], c.local[2]});
@@ -614,12 +733,21 @@ struct Stepper {
     return o;
   }
   __device__ void storeGroundDual(int i, const GroundDual &o) {
-    GroundContact<R> &c = E.s.gc[i];
-    c.id = o.id;
+    auto put = [&](GroundContact<R> &c) __attribute__((always_inline)) {
+      c.id = o.id;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      c.lambda[k] = o.lambda[k];
-      c.penalty[k] = o.penalty[k];
+      for (int k = 0; k < 3; ++k) {
+        c.lambda[k] = o.lambda[k];
+        c.penalty[k] = o.penalty[k];
+      }
+    };
+    if constexpr (Dense) {
+      if (i < kDenseContacts)
+        put(E.s.gc[i]);
+      else
+        put(common.list[i]);
+    } else {
+      put(E.s.gc[i]);
     }
   }
 
@@ -758,7 +886,7 @@ struct Stepper {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       // loads first, selects after: a conditional load would be a branch
-      const R c = fmad(-alpha, E.c0[k][ji], je.C[k]);
+      const R c = fmad(-alpha, C0(k, ji), je.C[k]);
       const R pen = E.s.penalty[k][ji], lam = E.s.lambda[k][ji];
       pr[k] = valid ? pen : R(0);
       fr[k] = valid ? fmad(pen, c, lam) : R(0);
@@ -795,7 +923,7 @@ struct Stepper {
     R limF[2], limK[2];
 #pragma unroll
     for (int k = 5; k < 7; ++k) {
-      const R c = fmad(-alpha, mn(E.c0[k][ji], R(0)), je.C[k]);
+      const R c = fmad(-alpha, mn(C0(k, ji), R(0)), je.C[k]);
       const R pen = E.s.penalty[k][ji];
       const R f = mn(fmad(pen, c, E.s.lambda[k][ji]), R(0));
       const bool on = limited && f < 0;
@@ -813,19 +941,19 @@ struct Stepper {
     } else {
       wrapAngle2(a0, a1, wTarget, delta);
     }
-    const R kp = E.s.kp[ji], maxT = E.s.maxTorque[ji];
-    R drive = fmad(kp, wTarget, -E.s.torque[ji]);
+    const R kp = Kp(ji), maxT = MaxTorque(ji);
+    R drive = fmad(kp, wTarget, -Torque(ji));
     const bool capped = maxT > 0;
     const R ks = capped && mabs(drive) >= maxT ? R(0) : kp;
     drive = capped ? clampv(drive, -maxT, maxT) : drive;
     R axisForce = implicitDrive ? drive : R(0), axisStiff = implicitDrive ? ks : R(0);
-    const R damping = E.s.damping[ji], armature = F.armature[ji], w0 = E.velocity0[ji];
+    const R damping = Damping(ji), armature = F.armature[ji], w0 = E.velocity0[ji];
     const R dh = fdivInv(damping, h, ih), ah = fdivInv(armature, h2, ih2);
     const R stiff = dh + ah;
     const bool damped = stiff > 0;
     axisForce += damped ? fmad(dh, delta, ah * fmad(-h, w0, delta)) : R(0);
     axisStiff += damped ? stiff : R(0);
-    const R fl = E.s.frictionloss[ji];
+    const R fl = FrictionLoss(ji);
     const R trial = fmad(E.s.penaltyF[ji], delta, E.s.lambdaF[ji]);
     axisForce += fl > 0 ? clampv(trial, -fl, fl) : R(0);
     axisStiff += fl > 0 && mabs(trial) < fl ? E.s.penaltyF[ji] : R(0);
@@ -842,8 +970,9 @@ struct Stepper {
   // Rows of ground contact `index` of body bi (kernel.cuh:915-931).  A
   // separating contact (f.z = 0) is stamped with zero force and stiffness;
   // with valid false the lever arm is zero as well (index clamped in range).
+  template <bool Far = false>
   __device__ void groundRows(Hess<R> &H, int bi, int index, bool valid) const {
-    const GroundContact<R> &c = E.s.gc[valid ? index : 0];
+    const auto &c = ground<Far>(valid ? index : 0);
     const int id = c.id;
     V3<R> ra = frotate(Q(bi), V3<R>{c.local[0], c.local[1], c.local[2]});
     V3<R> C = (X(bi) + ra) - V3<R>{c.anchor[0], c.anchor[1], R(0)};
@@ -910,11 +1039,13 @@ struct Stepper {
     for (int w = 0; w < GW; ++w)
       for (uint64_t m = E.gmask[w][bi]; m; m &= m - 1, ++nth)
         if ((nth + 1) % nParts == part % nParts)
-          groundRows(H, bi, 64 * w + __builtin_ctzll(m), true);
-    nth = 0;
-    for (uint32_t m = Pairs ? E.smask[bi] : 0u; m; m &= m - 1, ++nth)
-      if ((nth + 1) % nParts == part % nParts)
-        selfRows(H, bi, __builtin_ctz(m));
+          groundRows<Dense>(H, bi, 64 * w + __builtin_ctzll(m), true);
+    if constexpr (Pairs) {
+      nth = 0;
+      for (uint32_t m = E.smask[bi]; m; m &= m - 1, ++nth)
+        if ((nth + 1) % nParts == part % nParts)
+          selfRows(H, bi, __builtin_ctz(m));
+    }
   }
 
   // The float assembly: the inertia block, the lane's first hinge and (with
@@ -969,7 +1100,7 @@ struct Stepper {
             c0 | c1 << 8 | (adj0 + nParts) << 16 | adjEnd << 24};
   }
 
-  template <bool Ground, bool Given>
+  template <bool Ground, bool Given, bool Far = false>
   __device__ bool assembleFast(Hess<R> &H, int bi, bool implicitDrive, int part, int nParts,
                                SlotPlan sp, const JointEval *given) const {
     bool slow = false;
@@ -986,8 +1117,8 @@ struct Stepper {
     inertiaBlock<true>(H, bi, part, slow);
     hingeRows<true, Given>(H, bi, packed0, h0, implicitDrive, slow, given);
     if constexpr (Ground) {
-      groundRows(H, bi, sp.w1 & 255, (sp.w0 >> 25) & 1);
-      groundRows(H, bi, (sp.w1 >> 8) & 255, (sp.w0 >> 26) & 1);
+      groundRows<Far>(H, bi, sp.w1 & 255, (sp.w0 >> 25) & 1);
+      groundRows<Far>(H, bi, (sp.w1 >> 8) & 255, (sp.w0 >> 26) & 1);
     }
     for (int adj = adjNext; adj < adjEnd; adj += nParts)
       hingeRows<true>(H, bi, F.adj[adj], true, implicitDrive, slow);
@@ -1013,7 +1144,7 @@ struct Stepper {
       }
       while (__any(m != 0)) {
         const bool v = m != 0;
-        groundRows(H, bi, v ? __builtin_ctzll(m) : 0, v);
+        groundRows<Far>(H, bi, v ? __builtin_ctzll(m) : 0, v);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
           m = k < nParts ? m & (m - 1) : m;
@@ -1026,10 +1157,12 @@ struct Stepper {
           if ((!Ground || nth >= 2 * nParts) && nth % nParts == p0)
             groundRows(H, bi, 64 * w + __builtin_ctzll(g), true);
     }
-    int nth = 0;
-    for (uint32_t g = Pairs ? E.smask[bi] : 0u; g; g &= g - 1, ++nth)
-      if (nth % nParts == p0)
-        selfRows(H, bi, __builtin_ctz(g));
+    if constexpr (Pairs) {
+      int nth = 0;
+      for (uint32_t g = E.smask[bi]; g; g &= g - 1, ++nth)
+        if (nth % nParts == p0)
+          selfRows(H, bi, __builtin_ctz(g));
+    }
     return !slow;
   }
 
@@ -1057,39 +1190,52 @@ struct Stepper {
     const V3<R> x = X(bi);
     const Q4<R> q = Q(bi);
     Hess<R> H;
-    if (Pairs && finish) {
+    bool finished = false;
+    if constexpr (Pairs) {
+      if (finish) {
+        finished = true;
 #pragma unroll
-      for (int k = 0; k < 21; ++k)
-        H.h[k] = E.staged[part][k];
+        for (int k = 0; k < 21; ++k)
+          H.h[k] = E.staged[part][k];
 #pragma unroll
-      for (int k = 0; k < 6; ++k)
-        H.g[k] = E.staged[part][21 + k];
-      const int p0 = (part + nParts - 1) % nParts;
-      int nth = 0;
-      for (uint32_t g = E.earlyMask; g; g &= g - 1, ++nth)
-        if (nth % nParts == p0)
-          selfRows(H, bi, __builtin_ctz(g));
-    } else {
+        for (int k = 0; k < 6; ++k)
+          H.g[k] = E.staged[part][21 + k];
+        const int p0 = (part + nParts - 1) % nParts;
+        int nth = 0;
+        for (uint32_t g = E.earlyMask; g; g &= g - 1, ++nth)
+          if (nth % nParts == p0)
+            selfRows(H, bi, __builtin_ctz(g));
+      }
+    }
+    if (!finished) {
       bool done = false;
       if constexpr (sizeof(R) == sizeof(float)) {
         // Wave-uniform choices: with or without the straight-line contacts,
         // and the generic assembly for every lane when any lane fell outside
         // the fast forms.
-        const bool fast =
-            __any((sp.w0 >> 27) & 1)
-                ? assembleFast<true, Given>(H, bi, implicitDrive, part, nParts, sp, given)
-                : assembleFast<false, Given>(H, bi, implicitDrive, part, nParts, sp, given);
+        bool far = false;
+        if constexpr (Dense)
+          far = common.far;
+        bool fast;
+        if (Dense && far)
+          fast = assembleFast<true, Given, Dense>(H, bi, implicitDrive, part, nParts, sp, given);
+        else
+          fast = __any((sp.w0 >> 27) & 1)
+                     ? assembleFast<true, Given>(H, bi, implicitDrive, part, nParts, sp, given)
+                     : assembleFast<false, Given>(H, bi, implicitDrive, part, nParts, sp, given);
         done = !__any(!fast);
       }
       if (!done)
         assembleGeneric(H, bi, implicitDrive, part, nParts);
-      if (stage) {
+      if constexpr (Pairs) {
+        if (stage) {
 #pragma unroll
-        for (int k = 0; k < 21; ++k)
-          E.staged[part][k] = H.h[k];
+          for (int k = 0; k < 21; ++k)
+            E.staged[part][k] = H.h[k];
 #pragma unroll
-        for (int k = 0; k < 6; ++k)
-          E.staged[part][21 + k] = H.g[k];
+          for (int k = 0; k < 6; ++k)
+            E.staged[part][21 + k] = H.g[k];
+        }
       }
     }
     if constexpr (P >= 2) {

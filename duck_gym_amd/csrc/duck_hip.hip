@@ -276,6 +276,7 @@ class Batch final : public BatchBase {
   V3<R> *dPoints = nullptr;
   unsigned char *dStates = nullptr;
   hipEvent_t ready = nullptr;
+  int cus = 0; // compute units of the device
   void *dScratch = nullptr; // this device's `scratch`
   // Whether an environment's masses, inertia or friction may differ from the
   // model's (a reset with per-env extensions, an imported state): then every
@@ -292,6 +293,16 @@ class Batch final : public BatchBase {
   // code, launched for models that have none.
   static constexpr bool kPairless = sizeof(R) == sizeof(float) && L == 16;
 
+  // Whether a launch runs denseKernel: target controls, a float MicroDuck-sized
+  // model without body pairs, and more waves of four environments than the
+  // device has SIMDs (4096 environments on 256 compute units).  Below that line
+  // every wave has a SIMD of its own either way, and the full step's wave is the
+  // faster one (the standing workload at 4096: 90 against 98 us); above it the
+  // full step runs in rounds (6000: 170 us, the dense step 137).
+  bool dense(int waves, int mode) const {
+    return kPairless && host.pairs.empty() && mode == kTargetControls && waves > 4 * cus;
+  }
+
   void advance(unsigned char *states, int n, const void *targets, const void *forces,
                const void *motor, int substeps, double kp, double limit, hipStream_t s,
                int mode = -1) {
@@ -302,7 +313,11 @@ class Batch final : public BatchBase {
                   int(host.bodies.size()), int(host.joints.size()), int(host.shapes.size()),
                   int(host.pairs.size()), states == dStates && customBodies ? 1 : 0};
     if constexpr (kPairless) {
-      if (host.pairs.empty())
+      const int waves = (n + G - 1) / G;
+      if (dense(waves, mode))
+        denseKernel<R, B, J, CG, CS, L, PL>
+            <<<(waves + kDenseWaves - 1) / kDenseWaves, 64 * kDenseWaves, 0, s>>>(args);
+      else if (host.pairs.empty())
         advanceKernel<R, B, J, CG, CS, L, PL, false><<<(n + G - 1) / G, 64, 0, s>>>(args);
       else
         advanceKernel<R, B, J, CG, CS, L, PL><<<(n + G - 1) / G, 64, 0, s>>>(args);
@@ -345,6 +360,8 @@ public:
       hipCheck(hipDeviceSynchronize(), "initialize");
       hipCheck(hipEventCreateWithFlags(&ready, hipEventDisableTiming), "hipEventCreate");
       dScratch = referenceScratch(device);
+      hipCheck(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device),
+               "hipDeviceGetAttribute");
       record(0);
     } catch (...) {
       release();
@@ -646,8 +663,8 @@ public:
   }
   void layout(long long *out) const override;
   // Resources of the kernel this batch's duck_step (which = DUCK_KERNEL_STEP)
-  // or duck_servo_substep (DUCK_KERNEL_SERVO_SUBSTEP) launches -- the build
-  // without body-pair code for a model without pairs: VGPRs, static LDS and
+  // or duck_servo_substep (DUCK_KERNEL_SERVO_SUBSTEP) launches -- the dense
+  // step, or the build without body-pair code for a model without pairs: VGPRs, static LDS and
   // scratch per lane from the code object, resident workgroups per CU from
   // the runtime's occupancy calculator, lanes and environments per
   // workgroup, and workgroups per launch.
@@ -657,6 +674,7 @@ public:
             "kernel_info: unknown kernel");
     const bool pairless = kPairless && host.pairs.empty();
     const void *fn = nullptr;
+    int waves = 1; // of a workgroup
     if (which == DUCK_KERNEL_STEP)
       fn = reinterpret_cast<const void *>(&advanceKernel<R, B, J, CG, CS, L, PL>);
     else
@@ -666,15 +684,19 @@ public:
         fn = reinterpret_cast<const void *>(&advanceKernel<R, B, J, CG, CS, L, PL, false>);
       if (pairless && which == DUCK_KERNEL_SERVO_SUBSTEP)
         fn = reinterpret_cast<const void *>(&servoStepKernel<R, B, J, CG, CS, L, PL, false>);
+      if (which == DUCK_KERNEL_STEP && dense((count + G - 1) / G, kTargetControls)) {
+        fn = reinterpret_cast<const void *>(&denseKernel<R, B, J, CG, CS, L, PL>);
+        waves = kDenseWaves;
+      }
     }
     hipFuncAttributes a{};
     hipCheck(hipFuncGetAttributes(&a, fn), "hipFuncGetAttributes");
     int perCu = 0;
-    hipCheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, fn, 64, 0),
+    hipCheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, fn, 64 * waves, 0),
              "hipOccupancyMaxActiveBlocksPerMultiprocessor");
     const long long v[7] = {a.numRegs, static_cast<long long>(a.sharedSizeBytes),
-                            static_cast<long long>(a.localSizeBytes), perCu, 64, G,
-                            (count + G - 1) / G};
+                            static_cast<long long>(a.localSizeBytes), perCu, 64 * waves,
+                            G * waves, (count + G * waves - 1) / (G * waves)};
     for (int i = 0; i < 7; ++i)
       out[i] = v[i];
   }
