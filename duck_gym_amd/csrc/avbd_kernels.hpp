@@ -54,44 +54,30 @@ template <> __device__ __forceinline__ double swizzle16(double v) {
 }
 
 template <int L, class T> __device__ __forceinline__ T groupMax(T v) {
-  if constexpr (L == 16 || L == 32) {
-    T u = rowRor<8>(v);
+  static_assert(L == 16 || L == 32, "an environment has one or two DPP rows");
+  T u = rowRor<8>(v);
+  v = v > u ? v : u;
+  u = rowRor<4>(v);
+  v = v > u ? v : u;
+  u = rowRor<2>(v);
+  v = v > u ? v : u;
+  u = rowRor<1>(v);
+  v = v > u ? v : u;
+  if constexpr (L == 32) {
+    u = swizzle16(v);
     v = v > u ? v : u;
-    u = rowRor<4>(v);
-    v = v > u ? v : u;
-    u = rowRor<2>(v);
-    v = v > u ? v : u;
-    u = rowRor<1>(v);
-    v = v > u ? v : u;
-    if constexpr (L == 32) {
-      u = swizzle16(v);
-      v = v > u ? v : u;
-    }
-    return v;
-  } else {
-#pragma unroll
-    for (int o = L / 2; o > 0; o /= 2) {
-      T u = __shfl_xor(v, o, L);
-      v = v > u ? v : u;
-    }
-    return v;
   }
+  return v;
 }
 template <int L> __device__ __forceinline__ int groupOr(int v) {
-  if constexpr (L == 16 || L == 32) {
-    v |= rowRor<8>(v);
-    v |= rowRor<4>(v);
-    v |= rowRor<2>(v);
-    v |= rowRor<1>(v);
-    if constexpr (L == 32)
-      v |= swizzle16(v);
-    return v;
-  } else {
-#pragma unroll
-    for (int o = L / 2; o > 0; o /= 2)
-      v |= __shfl_xor(v, o, L);
-    return v;
-  }
+  static_assert(L == 16 || L == 32, "an environment has one or two DPP rows");
+  v |= rowRor<8>(v);
+  v |= rowRor<4>(v);
+  v |= rowRor<2>(v);
+  v |= rowRor<1>(v);
+  if constexpr (L == 32)
+    v |= swizzle16(v);
+  return v;
 }
 __device__ __forceinline__ int waveMaxInt(int v) {
 #pragma unroll

@@ -337,9 +337,9 @@ template <int N> __device__ __forceinline__ double rowRotate(double v) {
   return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
-// Lanes per block solve by default: one with up to 8 lanes per
-// environment, two with 16, four with 32.
-constexpr int defaultSolveLanes(int L) { return L >= 32 ? 4 : (L >= 16 ? 2 : 1); }
+// Lanes per block solve by default: two with 16 lanes per environment, four
+// with 32.
+constexpr int defaultSolveLanes(int L) { return L >= 32 ? 4 : 2; }
 
 // What a dense step holds outside its record: the launch's gains, the model's
 // channels (torque, frictionloss, damping; staged once per workgroup), and the

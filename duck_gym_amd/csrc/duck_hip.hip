@@ -289,9 +289,11 @@ class Batch final : public BatchBase {
   static int blocks64(int n) { return (n + 63) / 64; }
   // Blocks of the kernels that give an environment a lane per body slot.
   static int blocksPerBody(int n) { return (n + 64 / B - 1) / (64 / B); }
-  // The float MicroDuck-sized batch has a step compiled without body-pair
-  // code, launched for models that have none.
-  static constexpr bool kPairless = sizeof(R) == sizeof(float) && L == 16;
+  // The MicroDuck-sized batch has a step compiled without body-pair code,
+  // launched for models that have none (float64: in the default layout), and
+  // in float a dense one.
+  static constexpr bool kDense = sizeof(R) == sizeof(float) && L == 16;
+  static constexpr bool kPairless = kDense || (L == 16 && PL == 1);
 
   // Whether a launch runs denseKernel: target controls, a float MicroDuck-sized
   // model without body pairs, and more waves of four environments than the
@@ -300,7 +302,7 @@ class Batch final : public BatchBase {
   // faster one (the standing workload at 4096: 90 against 98 us); above it the
   // full step runs in rounds (6000: 170 us, the dense step 137).
   bool dense(int waves, int mode) const {
-    return kPairless && host.pairs.empty() && mode == kTargetControls && waves > 4 * cus;
+    return kDense && host.pairs.empty() && mode == kTargetControls && waves > 4 * cus;
   }
 
   void advance(unsigned char *states, int n, const void *targets, const void *forces,
@@ -314,10 +316,15 @@ class Batch final : public BatchBase {
                   int(host.pairs.size()), states == dStates && customBodies ? 1 : 0};
     if constexpr (kPairless) {
       const int waves = (n + G - 1) / G;
-      if (dense(waves, mode))
-        denseKernel<R, B, J, CG, CS, L, PL>
-            <<<(waves + kDenseWaves - 1) / kDenseWaves, 64 * kDenseWaves, 0, s>>>(args);
-      else if (host.pairs.empty())
+      if constexpr (kDense) {
+        if (dense(waves, mode)) {
+          denseKernel<R, B, J, CG, CS, L, PL>
+              <<<(waves + kDenseWaves - 1) / kDenseWaves, 64 * kDenseWaves, 0, s>>>(args);
+          launched("denseKernel");
+          return;
+        }
+      }
+      if (host.pairs.empty())
         advanceKernel<R, B, J, CG, CS, L, PL, false><<<(n + G - 1) / G, 64, 0, s>>>(args);
       else
         advanceKernel<R, B, J, CG, CS, L, PL><<<(n + G - 1) / G, 64, 0, s>>>(args);
@@ -684,6 +691,8 @@ public:
         fn = reinterpret_cast<const void *>(&advanceKernel<R, B, J, CG, CS, L, PL, false>);
       if (pairless && which == DUCK_KERNEL_SERVO_SUBSTEP)
         fn = reinterpret_cast<const void *>(&servoStepKernel<R, B, J, CG, CS, L, PL, false>);
+    }
+    if constexpr (kDense) {
       if (which == DUCK_KERNEL_STEP && dense((count + G - 1) / G, kTargetControls)) {
         fn = reinterpret_cast<const void *>(&denseKernel<R, B, J, CG, CS, L, PL>);
         waves = kDenseWaves;
@@ -754,13 +763,13 @@ const char *kMicroDuckJoints[14] = {
     "right_knee",      "right_ankle"};
 
 // MicroDuck-sized models (16 bodies and 14 hinges, the reference's
-// MicroDuckState, kernel.cuh:1098): float runs 4 environments per wave with two lanes
-// per block solve (16 lanes per env); double runs 8 environments per wave
-// with one lane per block solve, which keeps the reference's accumulation
-// order (DUCK_FLAG_SPLIT selects the float layout for double too).  Four
-// lanes per block solve (32 lanes per env, 20 KB of LDS per workgroup)
-// would let two waves share a SIMD only below 256 registers per lane, which
-// this kernel exceeds; with register spills it measured slower.
+// MicroDuckState, kernel.cuh:1098): 4 environments per wave with 16 lanes
+// each.  Float runs two lanes per block solve; double one, which keeps the
+// reference's accumulation order (DUCK_FLAG_SPLIT selects the float layout for
+// double too).  With 8 lanes per environment, and so two rounds over the
+// hinges and shapes, the double step held 1584 B of spills per lane and took
+// 418 us at 2048 standing environments, against 290 us (831 and 568 us at
+// 4096).
 template <class R>
 BatchBase *makeBatch(HostModel &&m, int n, double dt, int iterations, int device, bool split) {
   const int nb = m.bodies.size(), nj = m.joints.size(), ns = m.shapes.size(),
@@ -768,7 +777,7 @@ BatchBase *makeBatch(HostModel &&m, int n, double dt, int iterations, int device
   if (nb <= 16 && nj <= 14 && ns <= 16 && np <= 8 && m.groundCapacity <= 64) {
     if constexpr (sizeof(R) == sizeof(double))
       if (!split)
-        return new Batch<R, 16, 14, 64, 8, 8>(std::move(m), n, dt, iterations, device);
+        return new Batch<R, 16, 14, 64, 8, 16, 1>(std::move(m), n, dt, iterations, device);
     return new Batch<R, 16, 14, 64, 8, 16>(std::move(m), n, dt, iterations, device);
   }
   // The generic state: 32 bodies and hinges, 4 ground contacts for each of
