@@ -175,10 +175,11 @@ __device__ __forceinline__ void dmaChunks(const unsigned char *src, __attribute_
 // The blobs of a wave's environments into LDS, first round, as LDS DMA: the
 // group every step reads and writes (poses through the counts) with the first
 // kWarmContacts ground contacts as one range and, with `bodies`, the
-// reset-only group.  Environment g of the wave is e0 + g.
+// reset-only group.  Environment g of the wave is e0 + g, for the first `here`;
+// the records past them hold environment e0 (Fill) or stay as they are.
 constexpr int kWarmContacts = 8;
-template <class S, int G, bool Prefix = false, class Env>
-__device__ void loadHot(Env *envs, unsigned char *states, long long blobBytes, int e0, int count, int t,
+template <class S, int G, bool Prefix = false, bool Fill = false, class Env>
+__device__ void loadHot(Env *envs, unsigned char *states, long long blobBytes, int e0, int here, int t,
                         bool bodies) {
   constexpr int CGcap = int(sizeof(S::gc) / sizeof(S::gc[0]));
   constexpr int gcBytes = int(sizeof(decltype(S::gc[0])));
@@ -189,9 +190,9 @@ __device__ void loadHot(Env *envs, unsigned char *states, long long blobBytes, i
                 "copied groups are whole 16-byte chunks, group 1 starts on 128 bytes");
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    if (e0 + g >= count)
+    if (!Fill && g >= here)
       break;
-    const unsigned char *blob = states + blobBytes * (e0 + g);
+    const unsigned char *blob = states + blobBytes * (e0 + (g < here ? g : 0));
     auto *lds = (__attribute__((address_space(3))) unsigned char *)(&envs[g].s);
     dmaChunks<(warm - hot) / 16>(blob + hot, lds + hot, t);
     if (!Prefix && bodies) // (a record that holds the blob's prefix only has no such group)
@@ -593,7 +594,7 @@ template <class R> struct ServoArgs {
 template <class R, int B, int J, int CG, int CS, int L, int JPL, class Env>
 __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const DeviceModel<R> &M,
                                               const Frames<R, B, J> &F, Env &E, int e, int lane,
-                                              bool valid, int count, R (&ctl)[JPL][3]);
+                                              bool own, int count, R (&ctl)[JPL][3]);
 template <class R, int B, int J, int CG, int CS, class Env>
 __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const DeviceModel<R> &M, Env &E,
                                               int e);
@@ -683,7 +684,8 @@ __global__ void framesKernel(const DeviceModel<R> *model, Frames<R, B, J> *out) 
 }
 
 //
-// `block` is the wave's number: it advances environments block * G + g.
+// `block` is the wave's number: it advances environments block * per + g,
+// with per = args.perWave <= G (Dense: G).
 // Dense: the step of target controls of a model without body pairs with two
 // waves per SIMD -- kDenseWaves waves per workgroup, each on its own (they
 // share the Frames copy and meet once, after it has landed), on records that
@@ -724,8 +726,19 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   const V3<R> *points = static_cast<const V3<R> *>(args.points);
   const int t = Dense ? int(threadIdx.x % 64) : int(threadIdx.x), wave = Dense ? int(threadIdx.x / 64) : 0;
   const int lane = t % L, g = t / L;
-  const int e = block * G + g;
-  const bool valid = e < args.count;
+  // A wave with fewer than G environments runs its first one on the lane
+  // groups that are left, each on a record of its own, of which nothing is
+  // stored (`own` false).  A wave with whole rows of lanes masked off runs the
+  // same instructions slower: 64 standing environments, one to a wave, spend
+  // 4.5 k of 53.3 k quad-cycles waiting to issue, with the other rows working
+  // 0.5 k of 50.2 k (a launch's kernel 97 against 85 us, as with four
+  // environments to a wave; one environment, four steps: 337 -> 309 us).
+  const int per = Dense ? G : args.perWave, e0 = block * per;
+  constexpr bool Fill = !Dense;
+  const int here = args.count - e0 < per ? args.count - e0 : per;
+  const bool own = g < here;
+  const int e = Fill && !own ? e0 : e0 + g;
+  const bool valid = Fill || own;
   Env *envs = envsOf + wave * G;
   Env &E = envs[g];
   // (a model without body pairs: none of their code is compiled)
@@ -782,7 +795,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   }
   static_assert(L >= 4, "blob copies give each of the first three lanes an end word");
   static_assert(CS <= B, "the staged pair table holds B pairs");
-  loadHot<State, G, Dense>(envs, args.states, args.blobBytes, e - g, args.count, t, args.bodies != 0);
+  loadHot<State, G, Dense, Fill>(envs, args.states, args.blobBytes, e0, here, t, args.bodies != 0);
   if constexpr (Dense) {
     if (wave == 0 && t < J) {
 #pragma unroll
@@ -830,7 +843,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       massPattern |= (E.s.mass[b] > 0) != (F.mass[b] > 0);
   const bool defaultSchedule = groupOr<L>(massPattern) == 0;
   if constexpr (Servo)
-    servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, valid, args.count, ctl);
+    servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, own, args.count, ctl);
 
   // ---- controls (extension.cu:87-110 / kernel.cuh:448-466) ----
   int bad = 0;
@@ -1885,7 +1898,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     meet();
   }
   if constexpr (Servo)
-    if (valid && lane == 0)
+    if (own && lane == 0)
       servoEpilogue<R, B, J, CG, CS>(sv, M, E, e);
   // The colouring of an environment that stepped is the model's exactly when
   // no body took a fresh colour; it is written when the blob holds another.
@@ -1913,7 +1926,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       if (writeColours && lane < B)
         gs->colors[lane] = lane < nb ? M.colors[lane] : 0;
     }
-  } else if (valid) {
+  } else if (own) {
     storeEnv<State>(gs, E.s, lane, L, plan >> 8, (plan >> 1) & 3, writeColours);
   }
 }

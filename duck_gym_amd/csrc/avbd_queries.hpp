@@ -666,7 +666,7 @@ __global__ __launch_bounds__(64) void generalizedLoadsKernel(const DeviceModel<R
   const bool valid = e < count;
   const int nj = M.nj;
   auto &E = envs[g];
-  loadHot<State, G>(envs, states, blobBytes, e0, count, t, true);
+  loadHot<State, G>(envs, states, blobBytes, e0, count - e0, t, true);
   if (t < nj)
     jb[t] = M.jb[t];
   if (valid) {

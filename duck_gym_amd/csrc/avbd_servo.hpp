@@ -120,18 +120,20 @@ __global__ void servoKernel(DuckServo p, const DeviceModel<R> *model, unsigned c
 // listed parent first, the first lane runs it in hinge order), with its
 // per-body quantities in the step's per-step scratch, which the step fills
 // later; the first lane sums the supply in servoKernel's order.  The channels
-// go into `ctl`, where the motor step takes them.
+// go into `ctl`, where the motor step takes them.  A lane group that repeats
+// another's environment (`own` false) forms the same channels and stores
+// nothing: what it reads is read before the same wave's lanes write it.
 template <class R, int B, int J, int CG, int CS, int L, int JPL, class Env>
 __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const DeviceModel<R> &M,
                                               const Frames<R, B, J> &F, Env &E, int e, int lane,
-                                              bool valid, int count, R (&ctl)[JPL][3]) {
+                                              bool own, int count, R (&ctl)[JPL][3]) {
   static_assert(sizeof(RneaWork<R, B>) <= sizeof(R) * 20 * B, "the load pass fits x0 .. Iw");
   static_assert(3 * J < 7 * J - 1, "loads and supply fit c0");
   const int nj = M.nj, slots = sv.p.lag + 1;
   const size_t row = size_t(e) * nj, plane = size_t(count) * nj;
   R *loads = &E.c0[0][0];
   R delayed[JPL];
-  if (valid) {
+  {
     // bam_env.py:308-314: this substep's target into the ring (every slot
     // of a fresh ring), the target `lag` substeps old out
     const bool fresh = !sv.initialized[e];
@@ -143,34 +145,38 @@ __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const Devi
       if (j >= nj)
         continue;
       const R t = sv.target[row + j];
-      sv.history[size_t(sv.cursor) * plane + row + j] = t;
-      if (fresh)
-        for (int k = 0; k < slots; ++k)
-          sv.history[size_t(k) * plane + row + j] = t;
-      delayed[r] = sv.history[size_t(delayedSlot) * plane + row + j];
+      // (a slot written here is not read back)
+      const bool now = fresh || delayedSlot == sv.cursor;
+      delayed[r] = now ? t : sv.history[size_t(delayedSlot) * plane + row + j];
+      if (own) {
+        sv.history[size_t(sv.cursor) * plane + row + j] = t;
+        if (fresh)
+          for (int k = 0; k < slots; ++k)
+            sv.history[size_t(k) * plane + row + j] = t;
+      }
     }
   }
   auto &work = *reinterpret_cast<RneaWork<R, B> *>(&E.x0[0][0]);
   if (M.jointLevels > 0)
     rneaLoadsLanes<R, B, J, CG, CS, L>(M, E.s, sv.rootOffset + size_t(e) * 3, loads, work, F.b, lane,
-                                       valid);
-  if (valid) {
-    if (lane == 0) {
-      if (M.jointLevels == 0)
-        rneaLoadsIn<R, B, J, CG, CS>(M, E.s, sv.rootOffset + size_t(e) * 3, loads, work);
-      R total = 0;
-      for (int j = 0; j < nj; ++j)
-        total += mabs(sv.previousMotor[row + j]);
-      R supply = R(sv.p.vin) - R(sv.p.vin_drop_gain) * total;
-      supply = supply < R(sv.p.vin_min) ? R(sv.p.vin_min) : supply;
-      E.c0[6][J - 1] = supply;
+                                       true);
+  if (lane == 0) {
+    if (M.jointLevels == 0)
+      rneaLoadsIn<R, B, J, CG, CS>(M, E.s, sv.rootOffset + size_t(e) * 3, loads, work);
+    R total = 0;
+    for (int j = 0; j < nj; ++j)
+      total += mabs(sv.previousMotor[row + j]);
+    R supply = R(sv.p.vin) - R(sv.p.vin_drop_gain) * total;
+    supply = supply < R(sv.p.vin_min) ? R(sv.p.vin_min) : supply;
+    E.c0[6][J - 1] = supply;
+    if (own) {
       if (sv.supply)
         sv.supply[e] = supply;
       sv.initialized[e] = 1;
     }
   }
   __syncthreads();
-  if (valid) {
+  {
     StateView<R, B, J, CG, CS> view{M, E.s};
     const R supply = E.c0[6][J - 1];
 #pragma unroll
@@ -184,13 +190,15 @@ __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const Devi
       R applied, budget, damping, raw;
       xl330(sv.p, supply, delayed[r], position, velocity, sv.previousApplied[row + j], external,
             applied, budget, damping, raw);
-      if (sv.motor) {
+      if (own && sv.motor) {
         sv.motor[(row + j) * 3] = applied;
         sv.motor[(row + j) * 3 + 1] = budget;
         sv.motor[(row + j) * 3 + 2] = damping;
       }
-      sv.previousMotor[row + j] = raw;
-      sv.previousApplied[row + j] = applied;
+      if (own) {
+        sv.previousMotor[row + j] = raw;
+        sv.previousApplied[row + j] = applied;
+      }
       ctl[r][0] = applied;
       ctl[r][1] = budget;
       ctl[r][2] = damping;

@@ -40,6 +40,7 @@ struct StepArgs {
                       // first loads need only the kernel arguments
   int bodies;         // read the reset-only block (masses, inertia, friction)
                       // of each state; else they are the model's
+  int perWave;        // environments a wave advances (1 .. 64 / L)
 };
 
 DUCK_HD constexpr int tri(int i, int j) { return i * (i + 1) / 2 + j; }

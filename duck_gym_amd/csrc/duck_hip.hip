@@ -305,6 +305,25 @@ class Batch final : public BatchBase {
     return kDense && host.pairs.empty() && mode == kTargetControls && waves > 4 * cus;
   }
 
+  // Environments a wave of the full step advances in a launch of n.  The
+  // environments of a wave take each other's turns (contact rounds, body-pair
+  // queries, third colours, the double step's angle branches), so they get
+  // waves of their own while those are free.  Float waves that share a CU cost
+  // each other more than that (500 standing environments as 500, 250 and 125
+  // waves: 94.5, 90.8, 90.1 us; a sweep of 100 as 100, 50 and 25: 135, 139,
+  // 143 us), so they stop at one to a CU; in double the turns cost more (501
+  // environments as 501, 251 and 126 waves: 298, 323, 343 us), so those stop
+  // where every wave is still resident.
+  static constexpr int kResident =
+      int(160 * 1024 / (sizeof(Frames<R, B, J>) + G * sizeof(typename Stepper<R, B, J, CG, CS, L, PL>::Env)));
+  int perWave(int n) const {
+    const int waves = cus * (sizeof(R) == sizeof(float) ? 1 : kResident);
+    int per = 1;
+    while (per < G && (n + per - 1) / per > waves)
+      per *= 2;
+    return per;
+  }
+
   void advance(unsigned char *states, int n, const void *targets, const void *forces,
                const void *motor, int substeps, double kp, double limit, hipStream_t s,
                int mode = -1) {
@@ -313,7 +332,8 @@ class Batch final : public BatchBase {
     StepArgs args{dModel, dFrames, dPoints, states, blobBytes, n, targets, forces, motor,
                   substeps, mode, kp, limit,
                   int(host.bodies.size()), int(host.joints.size()), int(host.shapes.size()),
-                  int(host.pairs.size()), states == dStates && customBodies ? 1 : 0};
+                  int(host.pairs.size()), states == dStates && customBodies ? 1 : 0, perWave(n)};
+    const int blocks = (n + args.perWave - 1) / args.perWave;
     if constexpr (kPairless) {
       const int waves = (n + G - 1) / G;
       if constexpr (kDense) {
@@ -325,11 +345,11 @@ class Batch final : public BatchBase {
         }
       }
       if (host.pairs.empty())
-        advanceKernel<R, B, J, CG, CS, L, PL, false><<<(n + G - 1) / G, 64, 0, s>>>(args);
+        advanceKernel<R, B, J, CG, CS, L, PL, false><<<blocks, 64, 0, s>>>(args);
       else
-        advanceKernel<R, B, J, CG, CS, L, PL><<<(n + G - 1) / G, 64, 0, s>>>(args);
+        advanceKernel<R, B, J, CG, CS, L, PL><<<blocks, 64, 0, s>>>(args);
     } else {
-      advanceKernel<R, B, J, CG, CS, L, PL><<<(n + G - 1) / G, 64, 0, s>>>(args);
+      advanceKernel<R, B, J, CG, CS, L, PL><<<blocks, 64, 0, s>>>(args);
     }
     launched("advanceKernel");
   }
@@ -647,15 +667,16 @@ public:
     StepArgs args{dModel, dFrames, dPoints, dStates, blobBytes, count, nullptr, nullptr, nullptr,
                   1, kMotorControls, 0, 0,
                   nb, int(host.joints.size()), int(host.shapes.size()), int(host.pairs.size()),
-                  customBodies ? 1 : 0};
+                  customBodies ? 1 : 0, perWave(count)};
+    const int blocks = (count + args.perWave - 1) / args.perWave;
     wait(s);
     if constexpr (kPairless) {
       if (host.pairs.empty())
-        servoStepKernel<R, B, J, CG, CS, L, PL, false><<<(count + G - 1) / G, 64, 0, s>>>(args, sv);
+        servoStepKernel<R, B, J, CG, CS, L, PL, false><<<blocks, 64, 0, s>>>(args, sv);
       else
-        servoStepKernel<R, B, J, CG, CS, L, PL><<<(count + G - 1) / G, 64, 0, s>>>(args, sv);
+        servoStepKernel<R, B, J, CG, CS, L, PL><<<blocks, 64, 0, s>>>(args, sv);
     } else {
-      servoStepKernel<R, B, J, CG, CS, L, PL><<<(count + G - 1) / G, 64, 0, s>>>(args, sv);
+      servoStepKernel<R, B, J, CG, CS, L, PL><<<blocks, 64, 0, s>>>(args, sv);
     }
     launched("servoStepKernel");
     record(s);
@@ -703,9 +724,10 @@ public:
     int perCu = 0;
     hipCheck(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, fn, 64 * waves, 0),
              "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+    const int envs = waves > 1 ? G * waves : perWave(count);
     const long long v[7] = {a.numRegs, static_cast<long long>(a.sharedSizeBytes),
                             static_cast<long long>(a.localSizeBytes), perCu, 64 * waves,
-                            G * waves, (count + G * waves - 1) / (G * waves)};
+                            envs, (count + envs - 1) / envs};
     for (int i = 0; i < 7; ++i)
       out[i] = v[i];
   }

@@ -1,0 +1,85 @@
+"""Waves with fewer environments than they have room for: the lane groups left
+over repeat the wave's first environment and store nothing, so an environment
+steps bitwise the same with one, two or four to a wave, and a servo substep
+writes every row of its outputs exactly once."""
+
+import numpy as np
+import pytest
+import torch
+
+from duck_gym_amd import CudaBatch
+from duck_gym_amd.microduck import model_text
+from duck_gym_amd.servo import SYNTHETIC_SUPPLY, ServoLoop, servo_params
+
+pytestmark = pytest.mark.gpu
+
+DEV, DT, ITER = "cuda:0", 0.005, 10
+
+
+def _parts(fp64):
+    """A batch of four environments to a wave (the last one holding three),
+    and the same environments as two to a wave (the last one alone), one to a
+    wave, and three in all."""
+    waves = torch.cuda.get_device_properties(0).multi_processor_count * (2 if fp64 else 1)
+    return [slice(0, 2 * waves + 3), slice(0, waves + 1), slice(waves + 1, 2 * waves),
+            slice(2 * waves, 2 * waves + 3)]
+
+
+def _batches(pairs, fp64):
+    text, meta = model_text(self_contact=pairs)
+    parts = _parts(fp64)
+    dtype = torch.float64 if fp64 else torch.float32
+    batches = [CudaBatch.from_text(text, p.stop - p.start, DT, ITER, 0, fp64) for p in parts]
+    assert [b.kernel_info()["envs_per_workgroup"] for b in batches] == [4, 2, 1, 1]
+    rng, home = np.random.default_rng(11), np.array(meta["home"])
+    E = parts[0].stop
+    q, root = home + rng.uniform(-0.05, 0.05, (E, 14)), np.zeros((E, 6))
+    root[:, 3:5] = rng.uniform(-0.02, 0.02, (E, 2))
+    t = lambda a, p: torch.tensor(a[p], dtype=dtype, device=DEV)  # noqa: E731
+    for b, p in zip(batches, parts):
+        b.reset(torch.ones(p.stop - p.start, dtype=torch.bool, device=DEV), t(q, p), t(root, p))
+    return batches, parts, meta, home, rng, t
+
+
+def _same(outputs):
+    whole, *rest = outputs
+    for k, (w, *r) in enumerate(zip(whole, *rest)):
+        joined = torch.cat(r)
+        assert torch.equal(w, joined), (k, (w - joined).abs().max())
+
+
+@pytest.mark.parametrize("pairs,fp64", [(False, False), (True, False), (False, True), (True, True)])
+def test_environments_step_the_same_however_many_share_a_wave(pairs, fp64):
+    batches, parts, _, home, rng, t = _batches(pairs, fp64)
+    E = parts[0].stop
+    for substeps in (1, 3, 1, 2):
+        targets = home + rng.uniform(-0.2, 0.2, (E, 14))
+        forces = rng.uniform(-0.1, 0.1, (E, 3))
+        if substeps == 3:
+            targets[E - 1, 2] = np.nan  # refused: that environment fails
+        for b, p in zip(batches, parts):
+            b.step(t(targets, p), t(forces, p), substeps, 8.0, 0.0)
+        _same([b.state() for b in batches])
+    assert int(batches[0].state()[2][:, 5].sum()) == 1
+    motor = np.abs(rng.uniform(0, 0.1, (E, 14, 3)))
+    for b, p in zip(batches, parts):
+        b.step_motor(t(motor, p), t(np.zeros((E, 3)), p))
+        b.advance(2)
+    _same([(*b.state(), b.contact_forces(), b.contact_counts()) for b in batches])
+
+
+@pytest.mark.parametrize("lag,fp64", [(0, False), (2, False), (2, True)])
+def test_servo_substeps_are_the_same_however_many_share_a_wave(lag, fp64):
+    batches, parts, meta, home, rng, t = _batches(True, fp64)
+    feet = [meta["body_names"].index(n) for n in ("left_foot", "right_foot")]
+    loops = [ServoLoop(b, servo_params(**SYNTHETIC_SUPPLY, lag=lag), home, [0.0, 0.0, 0.01],
+                       root_principal_quat=meta["root_iquat"], feet=feet,
+                       foot_sites=[[0.01, 0.0, -0.006]] * 2, mean_velocity_tau=0.2) for b in batches]
+    for _ in range(3):
+        targets = home + rng.uniform(-0.2, 0.2, (parts[0].stop, 14))
+        for loop, p in zip(loops, parts):
+            loop.substeps(t(targets, p), 2)
+        _same([(*x.batch.state(), x.motor, x.previous_motor, x.previous_applied, x.initialized,
+                x.history.transpose(0, 1), x.gravity, x.lin_vel, x.contact_force, x.site_pos,
+                x.air_time, x.contact_time, x.self_contacts, x.self_penetration,
+                x.mean_velocity) for x in loops])
