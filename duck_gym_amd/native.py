@@ -257,12 +257,14 @@ class CudaBatch:
     def _stream(self):
         return ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
 
-    def _check(self, t, shape, dtype=None):
+    def _check(self, t, shape, dtype=None, stream=None):
+        """The pointer of `t`, checked and recorded on `stream` (default: the
+        current one; a call with many tensors looks it up once)."""
         dtype = self.dtype if dtype is None else dtype
         if not (isinstance(t, torch.Tensor) and t.is_cuda and t.device.index == self.device.index
                 and t.dtype == dtype and t.is_contiguous() and list(t.shape) == list(shape)):
             raise RuntimeError("Invalid CUDA tensor device/dtype/shape/contiguity")
-        t.record_stream(torch.cuda.current_stream(self.device))
+        t.record_stream(torch.cuda.current_stream(self.device) if stream is None else stream)
         return ctypes.c_void_p(t.data_ptr())
 
     def _empty(self, *shape):
@@ -407,25 +409,29 @@ class CudaBatch:
                       self_penetration=None, gravity=None, angular_velocity=None,
                       linear_velocity=None, origin_velocity=None, foot_forces=None,
                       site_positions=None, site_velocities=None, air_time=None,
-                      contact_time=None, mean_velocity=None, mean_velocity_alpha=0.0):
+                      contact_time=None, mean_velocity=None, mean_velocity_alpha=0.0,
+                      count=1):
         """One fused BAM substep (include/duck_hip.h duck_servo_substep): the
         servo, the motor step with zero root force, the self-contact maxima,
         the refresh() quantities and, with `mean_velocity` [E,3], the
         mean-velocity filter mean += alpha (origin velocity - mean)
         (bam_env.py:343-345), in one launch.  Outputs are written into the
-        tensors given (any may be None); in/out tensors are updated in place."""
+        tensors given (any may be None); in/out tensors are updated in place.
+        `count` of them run with the same buffers, the history's cursor moving
+        on by one slot each; the buffers are looked over once (some 20 tensors:
+        as long on the host as a substep of 4096 environments on the GPU)."""
         E, J = self.num_envs, self.num_joints
         F = len(feet)
         if F > MAX_FEET:
             raise RuntimeError("servo substep: invalid foot count")
-        io = DuckServoSubstep()
-        io.target = self._check(target, [E, J]).value
-        io.history = self._check(history, [int(params.lag) + 1, E, J]).value
-        io.cursor = int(cursor)
-        io.initialized = self._check(initialized, [E], torch.bool).value
-        io.root_offset = self._check(root_offset, [E, 3]).value
-        io.previous_motor = self._check(previous_motor, [E, J]).value
-        io.previous_applied = self._check(previous_applied, [E, J]).value
+        io, slots = DuckServoSubstep(), int(params.lag) + 1
+        stream = torch.cuda.current_stream(self.device)
+        io.target = self._check(target, [E, J], None, stream).value
+        io.history = self._check(history, [slots, E, J], None, stream).value
+        io.initialized = self._check(initialized, [E], torch.bool, stream).value
+        io.root_offset = self._check(root_offset, [E, 3], None, stream).value
+        io.previous_motor = self._check(previous_motor, [E, J], None, stream).value
+        io.previous_applied = self._check(previous_applied, [E, J], None, stream).value
         for name, t, shape in (("motor", motor, [E, J, 3]), ("supply", supply, [E]),
                                ("self_contacts", self_contacts, [E]),
                                ("self_penetration", self_penetration, [E]),
@@ -438,8 +444,8 @@ class CudaBatch:
                                ("site_velocities", site_velocities, [E, F, 3]),
                                ("air_time", air_time, [E, F]), ("contact_time", contact_time, [E, F]),
                                ("mean_velocity", mean_velocity, [E, 3])):
-            ptr = self._ptr(t, shape)
-            setattr(io, name, None if ptr is None else ptr.value)
+            if t is not None:
+                setattr(io, name, self._check(t, shape, None, stream).value)
         io.mean_velocity_alpha = float(mean_velocity_alpha)
         for k in range(4):
             io.root_principal_quat[k] = float(root_principal_quat[k])
@@ -449,11 +455,13 @@ class CudaBatch:
             io.foot_bodies[f] = int(feet[f])
             for k in range(3):
                 io.foot_sites[f][k] = float(sites[f][k])
+        launch, raw = library().duck_servo_substep, ctypes.c_void_p(stream.cuda_stream)
         with torch.cuda.device(self.device):
-            code = library().duck_servo_substep(self._h, ctypes.byref(params), ctypes.byref(io),
-                                                self._stream())
-        if code:
-            _raise(code, "servo_substep")
+            for k in range(count):
+                io.cursor = int(cursor) if k == 0 else (int(cursor) + k) % slots
+                code = launch(self._h, ctypes.byref(params), ctypes.byref(io), raw)
+                if code:
+                    _raise(code, "servo_substep")
 
     def task_obs_dim(self, task):
         return int(library().duck_task_obs_dim(ctypes.byref(task), self.num_joints))

@@ -188,8 +188,11 @@ class ServoLoop:
         target = target.contiguous()
         self.self_contacts.zero_()
         self.self_penetration.zero_()
-        for _ in range(count):
-            if self.fused:
+        if self.fused:
+            # without a callback nothing can change between the substeps: one
+            # call for all of them
+            each = 1 if substep_callback is not None else count
+            for _ in range(0, count, max(each, 1)):
                 self.batch.servo_substep(
                     self.params, target, self.history, self.cursor, self.initialized,
                     self.root_offset, self.previous_motor, self.previous_applied,
@@ -201,11 +204,12 @@ class ServoLoop:
                     site_positions=self.site_pos, site_velocities=self.site_vel,
                     air_time=self.air_time, contact_time=self.contact_time,
                     mean_velocity=self.mean_velocity if self.mean_velocity_tau else None,
-                    mean_velocity_alpha=self.mean_alpha)
-                self.cursor = (self.cursor + 1) % (self.params.lag + 1)
+                    mean_velocity_alpha=self.mean_alpha, count=each)
+                self.cursor = (self.cursor + each) % (self.params.lag + 1)
                 if substep_callback is not None:
                     substep_callback(self)
-                continue
+            return
+        for _ in range(count):
             motor = self.batch.servo(self.params, target, self.history, self.cursor,
                                      self.initialized, self.root_offset, self.previous_motor,
                                      self.previous_applied)
