@@ -237,16 +237,17 @@ enum DriveWrite { kWriteNoDrive = 0, kWriteDrive = 1, kWriteMotorDrive = 2 };
 // group 1, by what the launch set) through the live ground contacts as one range,
 // the live body contacts, and the drive parameters (all, the motor-written
 // three, or none) and the colouring where they changed.  Mass, inertia and
-// friction only change on reset.
+// friction only change on reset.  `ngc` and `nsc`: the contacts written.
 template <class S>
-__device__ void storeEnv(S *dst, const S &src, int lane, int L, int from, int driveWrite, bool colours) {
+__device__ void storeEnv(S *dst, const S &src, int lane, int L, int from, int driveWrite, bool colours,
+                         int ngc, int nsc) {
   constexpr int header = int(headerBytes<S>() / 4);
   constexpr int gcWords = int(sizeof(decltype(S::gc[0])) / 4);
   constexpr int scStart = int(offsetof(S, sc) / 4), scWords = int(sizeof(decltype(S::sc[0])) / 4);
   unsigned *d = reinterpret_cast<unsigned *>(dst);
   const unsigned *s = reinterpret_cast<const unsigned *>(&src);
-  copyWords<16>(d, s, from, header + src.ngc * gcWords, lane, L);
-  copyWords<4>(d, s, scStart, scStart + src.nsc * scWords, lane, L);
+  copyWords<16>(d, s, from, header + ngc * gcWords, lane, L);
+  copyWords<4>(d, s, scStart, scStart + nsc * scWords, lane, L);
   if (driveWrite != kWriteNoDrive)
     copyWords<4>(d, s, int((driveWrite == kWriteDrive ? driveBegin<S>() : motorBegin<S>()) / 4),
                  int(driveEnd<S>() / 4), lane, L);
@@ -588,16 +589,49 @@ template <class R> struct ServoArgs {
   R meanAlpha;
 };
 
+// What a lane of the servo substep reads of the servo's buffers, loaded with
+// the controls so that its latency overlaps the staging: its hinges' target,
+// delayed slot of the history, previous raw and applied torque, whether the
+// environment's history is fresh, and (lanes 0 to 2) the root offset.
+template <class R, int JPL> struct ServoIn {
+  R target[JPL], history[JPL], motor[JPL], applied[JPL], offset;
+  bool fresh;
+};
+template <class R> __device__ __forceinline__ int delayedSlot(const ServoArgs<R> &sv) {
+  const int slots = sv.p.lag + 1;
+  return ((sv.cursor - sv.p.lag) % slots + slots) % slots;
+}
+template <int L, class R, int JPL>
+__device__ __forceinline__ void loadServo(const ServoArgs<R> &sv, int e, int lane, int nj, int count,
+                                          ServoIn<R, JPL> &in) {
+  const size_t row = size_t(e) * nj, plane = size_t(count) * nj;
+  const R *slot = sv.history + size_t(delayedSlot(sv)) * plane;
+#pragma unroll
+  for (int r = 0; r < JPL; ++r) {
+    const int j = lane + r * L;
+    in.target[r] = in.history[r] = in.motor[r] = in.applied[r] = 0;
+    if (j >= nj)
+      continue;
+    in.target[r] = sv.target[row + j];
+    in.history[r] = slot[row + j];
+    in.motor[r] = sv.previousMotor[row + j];
+    in.applied[r] = sv.previousApplied[row + j];
+  }
+  in.offset = lane < 3 ? sv.rootOffset[size_t(e) * 3 + lane] : R(0);
+  in.fresh = !sv.initialized[e];
+}
+
 // The servo substep's prologue (the motor channels of this substep into
 // `ctl`) and epilogue (statistics and refresh quantities), defined with the
 // actuator model in avbd_servo.hpp.
 template <class R, int B, int J, int CG, int CS, int L, int JPL, class Env>
 __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const DeviceModel<R> &M,
                                               const Frames<R, B, J> &F, Env &E, int e, int lane,
-                                              bool own, int count, R (&ctl)[JPL][3]);
-template <class R, int B, int J, int CG, int CS, class Env>
+                                              bool own, int count, int sub, ServoIn<R, JPL> &in,
+                                              R (&ctl)[JPL][3]);
+template <class R, int B, int J, int CG, int CS, int L, class Env>
 __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const DeviceModel<R> &M, Env &E,
-                                              int e);
+                                              int e, int lane);
 
 // Per-launch step: controls, `substeps` physics steps, write-back; with
 // Servo, the controls are the motor channels of one servo substep and the
@@ -768,6 +802,9 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     defs[r][1] = M.frictionloss[jc];
     defs[r][2] = M.damping[jc];
   }
+  ServoIn<R, JPL> servoIn{};
+  if constexpr (Servo)
+    loadServo<L>(sv, e, lane, nj, args.count, servoIn);
   if (!Servo && valid && lane < 3 && args.motorMode != kHeldControls)
     fin = static_cast<const R *>(args.forces)[size_t(e) * 3 + lane];
 
@@ -842,10 +879,17 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     for (int b = lane; b < nb; b += L)
       massPattern |= (E.s.mass[b] > 0) != (F.mass[b] > 0);
   const bool defaultSchedule = groupOr<L>(massPattern) == 0;
-  if constexpr (Servo)
-    servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, own, args.count, ctl);
-
   // ---- controls (extension.cu:87-110 / kernel.cuh:448-466) ----
+  // (once per launch; in a servo launch before every substep, with the
+  // channels its prologue forms)
+  bool active = false, ran = false;
+  // What the blob's drive parameters and colouring hold before this launch
+  // (read before any lane rewrites the stamps).
+  int driveWrite = kWriteNoDrive;
+  int writeFrom = int(hotBegin<State>() / 4);
+  const int driveIn = valid ? E.s.drive : kDriveOther;
+  const bool modelColoursIn = valid && E.s.modelColours != 0;
+  auto setControls = [&]() __attribute__((always_inline)) {
   int bad = 0;
   if (valid && args.motorMode != kHeldControls) {
 #pragma unroll
@@ -865,13 +909,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   }
   bad = groupOr<L>(bad);
   meet();
-  bool active = false;
-  // What the blob's drive parameters and colouring hold before this launch
-  // (read before any lane rewrites the stamps).
-  int driveWrite = kWriteNoDrive;
-  int writeFrom = int(hotBegin<State>() / 4);
-  const int driveIn = valid ? E.s.drive : kDriveOther;
-  const bool modelColoursIn = valid && E.s.modelColours != 0;
+  active = false;
   if (valid) {
     if (args.motorMode == kHeldControls) {
       // State::advance (kernel.cuh:421-443): the controls in the state as
@@ -938,7 +976,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       E.s.failed = 1;
     }
   }
-  const bool ran = active;
+  ran = ran || active;
   // an environment that steps rewrites its diagnostics (and its targets and
   // force, set or read above)
   if (ran)
@@ -946,7 +984,7 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   // the write-back's plan waits in LDS, not in registers across the solve
   if (valid && lane == 0)
     E.writeback = (modelColoursIn ? 1 : 0) | driveWrite << 1 | writeFrom << 8;
-  if (ran && lane == 0) {
+  if (active && lane == 0) {
     // the step's diagnostics start afresh (slots 6 and 7 unused, zero)
     for (int k = 0; k < 8; ++k) {
       E.stepDiag[k] = 0;
@@ -954,6 +992,9 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     }
   }
   meet();
+  };
+  if constexpr (!Servo)
+    setControls();
 
   Step stp{M, points, F, E, lane, {}};
   if constexpr (Dense)
@@ -974,9 +1015,29 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   const int slot = P == 1 ? lane : (lane & 7) + 8 * (lane / (8 * P));
   const R h = M.dt, alpha = M.alpha, gamma = M.gamma, ag = alpha * gamma;
 
-  for (int sub = 0; sub < args.substeps; ++sub) {
-    if (!__any(active))
-      break;
+  // (a servo launch ends every substep, also one that no environment steps,
+  // at the top of the next round; it writes back as many contacts as any of
+  // its substeps had, as a launch each would have)
+  int mostGround = 0, mostSelf = 0;
+  for (int sub = 0; sub < args.substeps + (Servo ? 1 : 0); ++sub) {
+    if constexpr (Servo) {
+      if (sub > 0 && own) {
+        servoEpilogue<R, B, J, CG, CS, L>(sv, M, E, e, lane);
+        mostGround = mostGround > E.s.ngc ? mostGround : E.s.ngc;
+        mostSelf = mostSelf > E.s.nsc ? mostSelf : E.s.nsc;
+      }
+      __syncthreads();
+      if (sub == args.substeps)
+        break;
+      servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, own, args.count, sub, servoIn, ctl);
+      setControls();
+    }
+    if (!__any(active)) {
+      if constexpr (Servo)
+        continue;
+      else
+        break;
+    }
     // ---------------- detection: body-body pairs (kernel.cuh:656-722) ----
     // (before the ground manifolds, so that the narrow phase does not hold
     // the ground passes' warm-start registers)
@@ -1897,9 +1958,6 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     meet();
     meet();
   }
-  if constexpr (Servo)
-    if (own && lane == 0)
-      servoEpilogue<R, B, J, CG, CS>(sv, M, E, e);
   // The colouring of an environment that stepped is the model's exactly when
   // no body took a fresh colour; it is written when the blob holds another.
   const int plan = valid ? E.writeback : 0;
@@ -1927,7 +1985,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         gs->colors[lane] = lane < nb ? M.colors[lane] : 0;
     }
   } else if (own) {
-    storeEnv<State>(gs, E.s, lane, L, plan >> 8, (plan >> 1) & 3, writeColours);
+    storeEnv<State>(gs, E.s, lane, L, plan >> 8, (plan >> 1) & 3, writeColours, Servo ? mostGround : E.s.ngc,
+                    Servo ? mostSelf : E.s.nsc);
   }
 }
 
@@ -1957,8 +2016,15 @@ __global__ __launch_bounds__(64 * kDenseWaves, 2) __attribute__((aligned(32768))
       args, none, xcdBlock(blockIdx.x, gridDim.x) * kDenseWaves + int(threadIdx.x / 64));
 }
 
-// One servo substep per launch (bam_env.py:307-337 with refresh()), on a
-// 32 KiB boundary like advanceKernel.
+// Servo substeps (bam_env.py:307-337 with refresh()), on a 32 KiB boundary
+// like advanceKernel.  Bound, as the step, by the dependent chains of the
+// slowest wave; what the servo adds waits for memory, so its buffers are read
+// with the controls, ahead of the staging, and the substeps of a control step
+// run in one launch (no staging and write-back between them, and a wave that
+// is slow in one substep holds up no other before the last).  A control step
+// of four substeps and a state, 4096 environments: 534 -> 527 us with a launch
+// each before, 662 -> 647 us where some robots have fallen; a launch each with
+// the buffers read where they were used 690 us there.
 template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true>
 __global__ __launch_bounds__(64) __attribute__((aligned(32768))) void servoStepKernel(StepArgs args,
                                                                                    ServoArgs<R> servo) {

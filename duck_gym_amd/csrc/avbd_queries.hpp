@@ -488,8 +488,9 @@ DUCK_HD void rneaLoads(const DeviceModel<R> &M, const EnvState<R, B, J, CG, CS> 
 // workgroup calls it (barriers); `valid` lanes work.  The hinges' frames are
 // read once, ahead of the levels, and `jb` is the caller's LDS copy of the
 // hinges' child bodies: a level then waits for LDS, not for the model in
-// global memory (the fused servo substep 110.7 -> 108.4 us).
-template <class R, int B, int J, int CG, int CS, int L>
+// global memory (the fused servo substep 110.7 -> 108.4 us).  Drive: with the
+// actuator column.
+template <class R, int B, int J, int CG, int CS, int L, bool Drive = true>
 __device__ __forceinline__ void rneaLoadsLanes(const DeviceModel<R> &M,
                                                const EnvState<R, B, J, CG, CS> &s, const R *off,
                                                R *o, RneaWork<R, B> &work, const int *jb, int lane,
@@ -520,7 +521,7 @@ __device__ __forceinline__ void rneaLoadsLanes(const DeviceModel<R> &M,
     jA[r] = in ? M.ja[j] : 0;
     jB[r] = in ? M.jb[j] : 0;
     jAxis[r] = jRb[r] = V3<R>{0, 0, 0};
-    if (in) {
+    if (Drive && in) {
       R motor = s.torque[j] - s.kp[j] * wrapAngle(v.angle(j) - s.target[j]);
       o[3 * j + 2] = s.maxTorque[j] > 0 ? clampv(motor, -s.maxTorque[j], s.maxTorque[j]) : motor;
     }

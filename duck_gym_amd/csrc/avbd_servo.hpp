@@ -119,90 +119,94 @@ __global__ void servoKernel(DuckServo p, const DeviceModel<R> *model, unsigned c
 // tree level at a time (rneaLoadsLanes; for a model whose hinges are no tree
 // listed parent first, the first lane runs it in hinge order), with its
 // per-body quantities in the step's per-step scratch, which the step fills
-// later; the first lane sums the supply in servoKernel's order.  The channels
+// later; every lane sums the supply in servoKernel's order.  The channels
 // go into `ctl`, where the motor step takes them.  A lane group that repeats
 // another's environment (`own` false) forms the same channels and stores
-// nothing: what it reads is read before the same wave's lanes write it.
+// nothing: what it reads (loadServo) is read before the same wave's lanes
+// write it.
 template <class R, int B, int J, int CG, int CS, int L, int JPL, class Env>
 __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const DeviceModel<R> &M,
                                               const Frames<R, B, J> &F, Env &E, int e, int lane,
-                                              bool own, int count, R (&ctl)[JPL][3]) {
+                                              bool own, int count, int sub, ServoIn<R, JPL> &in,
+                                              R (&ctl)[JPL][3]) {
   static_assert(sizeof(RneaWork<R, B>) <= sizeof(R) * 20 * B, "the load pass fits x0 .. Iw");
-  static_assert(3 * J < 7 * J - 1, "loads and supply fit c0");
+  static_assert(4 * J + 3 <= 7 * J, "loads, previous torques and root offset fit c0");
   const int nj = M.nj, slots = sv.p.lag + 1;
   const size_t row = size_t(e) * nj, plane = size_t(count) * nj;
-  R *loads = &E.c0[0][0];
+  R *loads = &E.c0[0][0], *previous = loads + 3 * J, *offset = loads + 4 * J;
   R delayed[JPL];
-  {
-    // bam_env.py:308-314: this substep's target into the ring (every slot
-    // of a fresh ring), the target `lag` substeps old out
-    const bool fresh = !sv.initialized[e];
-    const int delayedSlot = ((sv.cursor - sv.p.lag) % slots + slots) % slots;
+  // bam_env.py:308-314: this substep's target into the ring (every slot
+  // of a fresh ring), the target `lag` substeps old out.  Slots that this
+  // launch has written hold its target and are not read back, so no lane
+  // reads what another writes.
+  const int cursor = (sv.cursor + sub) % slots;
+  const bool now = in.fresh || sub >= sv.p.lag;
 #pragma unroll
-    for (int r = 0; r < JPL; ++r) {
-      const int j = lane + r * L;
-      delayed[r] = 0;
-      if (j >= nj)
-        continue;
-      const R t = sv.target[row + j];
-      // (a slot written here is not read back)
-      const bool now = fresh || delayedSlot == sv.cursor;
-      delayed[r] = now ? t : sv.history[size_t(delayedSlot) * plane + row + j];
-      if (own) {
-        sv.history[size_t(sv.cursor) * plane + row + j] = t;
-        if (fresh)
-          for (int k = 0; k < slots; ++k)
-            sv.history[size_t(k) * plane + row + j] = t;
-      }
+  for (int r = 0; r < JPL; ++r) {
+    const int j = lane + r * L;
+    delayed[r] = in.target[r];
+    if (j >= nj)
+      continue;
+    if (!now)
+      delayed[r] = sub == 0 ? in.history[r] : sv.history[size_t((cursor + 1) % slots) * plane + row + j];
+    previous[j] = mabs(in.motor[r]);
+    if (own) {
+      sv.history[size_t(cursor) * plane + row + j] = in.target[r];
+      if (in.fresh && sub == 0)
+        for (int k = 0; k < slots; ++k)
+          sv.history[size_t(k) * plane + row + j] = in.target[r];
     }
   }
+  if (lane < 3)
+    offset[lane] = in.offset;
+  if (own && lane == 0)
+    sv.initialized[e] = 1;
   auto &work = *reinterpret_cast<RneaWork<R, B> *>(&E.x0[0][0]);
-  if (M.jointLevels > 0)
-    rneaLoadsLanes<R, B, J, CG, CS, L>(M, E.s, sv.rootOffset + size_t(e) * 3, loads, work, F.b, lane,
-                                       true);
-  if (lane == 0) {
-    if (M.jointLevels == 0)
-      rneaLoadsIn<R, B, J, CG, CS>(M, E.s, sv.rootOffset + size_t(e) * 3, loads, work);
-    R total = 0;
-    for (int j = 0; j < nj; ++j)
-      total += mabs(sv.previousMotor[row + j]);
-    R supply = R(sv.p.vin) - R(sv.p.vin_drop_gain) * total;
-    supply = supply < R(sv.p.vin_min) ? R(sv.p.vin_min) : supply;
-    E.c0[6][J - 1] = supply;
-    if (own) {
-      if (sv.supply)
-        sv.supply[e] = supply;
-      sv.initialized[e] = 1;
-    }
+  if (M.jointLevels > 0) {
+    rneaLoadsLanes<R, B, J, CG, CS, L, false>(M, E.s, offset, loads, work, F.b, lane, true);
+  } else {
+    __syncthreads();
+    if (lane == 0)
+      rneaLoadsIn<R, B, J, CG, CS>(M, E.s, offset, loads, work);
   }
   __syncthreads();
-  {
-    StateView<R, B, J, CG, CS> view{M, E.s};
-    const R supply = E.c0[6][J - 1];
+  R total = 0;
+  for (int j = 0; j < nj; ++j)
+    total += previous[j];
+  R supply = R(sv.p.vin) - R(sv.p.vin_drop_gain) * total;
+  supply = supply < R(sv.p.vin_min) ? R(sv.p.vin_min) : supply;
+  if (own && lane == 0 && sv.supply)
+    sv.supply[e] = supply;
+  StateView<R, B, J, CG, CS> view{M, E.s};
+  auto frame = [](const auto &a, int j) { return V3<R>{a[0][j], a[1][j], a[2][j]}; };
 #pragma unroll
-    for (int r = 0; r < JPL; ++r) {
-      const int j = lane + r * L;
-      if (j >= nj)
-        continue;
-      R position = view.angle(j);
-      R velocity = dot(view.W(M.jb[j]) - view.W(M.ja[j]), rotate(view.Q(M.ja[j]), view.mv(M.axisA, j)));
-      R external = -loads[3 * j] + loads[3 * j + 1];
-      R applied, budget, damping, raw;
-      xl330(sv.p, supply, delayed[r], position, velocity, sv.previousApplied[row + j], external,
-            applied, budget, damping, raw);
-      if (own && sv.motor) {
+  for (int r = 0; r < JPL; ++r) {
+    const int j = lane + r * L;
+    if (j >= nj)
+      continue;
+    const int a = F.a[j], b = F.b[j];
+    const Q4<R> qa = view.Q(a), qb = view.Q(b);
+    const V3<R> axisA = frame(F.axisA, j);
+    R position = hingeAngle(qa, qb, axisA, frame(F.tangentA, j), frame(F.tangentB, j));
+    R velocity = dot(view.W(b) - view.W(a), rotate(qa, axisA));
+    R external = -loads[3 * j] + loads[3 * j + 1];
+    R applied, budget, damping, raw;
+    xl330(sv.p, supply, delayed[r], position, velocity, in.applied[r], external, applied, budget,
+          damping, raw);
+    if (own) {
+      if (sv.motor) {
         sv.motor[(row + j) * 3] = applied;
         sv.motor[(row + j) * 3 + 1] = budget;
         sv.motor[(row + j) * 3 + 2] = damping;
       }
-      if (own) {
-        sv.previousMotor[row + j] = raw;
-        sv.previousApplied[row + j] = applied;
-      }
-      ctl[r][0] = applied;
-      ctl[r][1] = budget;
-      ctl[r][2] = damping;
+      sv.previousMotor[row + j] = raw;
+      sv.previousApplied[row + j] = applied;
     }
+    in.motor[r] = raw;
+    in.applied[r] = applied;
+    ctl[r][0] = applied;
+    ctl[r][1] = budget;
+    ctl[r][2] = damping;
   }
   __syncthreads(); // the load pass's scratch is the step's
 }
@@ -210,35 +214,43 @@ __device__ __forceinline__ void servoPrologue(const ServoArgs<R> &sv, const Devi
 // torch.maximum: NaN when either operand is NaN.
 template <class R> DUCK_HD R maximumNan(R a, R b) { return a != a || b != b ? R(NAN) : (a > b ? a : b); }
 
-// The end of the servo substep, on the environment's first lane after the
-// motor step: self_contact_stats (selfContactStatsKernel's loop) folded into
+// The end of the servo substep, after the motor step.  On the environment's
+// first lane: self_contact_stats (selfContactStatsKernel's loop) folded into
 // the running maxima (bam_env.py:333-335), then refresh() (bam_env.py:128-
-// 155) on the new state: gravity and velocities in the root frame, the
-// ground contact force on each foot (contactForcesKernel's sums), the foot
-// sites, the mean-velocity filter (bam_env.py:343-345) and the air/contact
-// timers.
-template <class R, int B, int J, int CG, int CS, class Env>
+// 155) on the new state: gravity and velocities in the root frame and the
+// mean-velocity filter (bam_env.py:343-345).  On a lane per foot: the ground
+// contact force on it (contactForcesKernel's sums), its site and the
+// air/contact timers.  What is read of the buffers is read first, in one
+// round trip.
+template <class R, int B, int J, int CG, int CS, int L, class Env>
 __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const DeviceModel<R> &M, Env &E,
-                                              int e) {
+                                              int e, int lane) {
+  static_assert(DUCK_MAX_FEET <= L, "a lane per foot");
   auto &s = E.s;
   StateView<R, B, J, CG, CS> v{M, s};
-  R n = 0, depthMax = 0;
-  for (int i = 0; i < s.nsc; ++i) {
-    const auto &c = s.sc[i];
-    int a = scBody(c.id), b = scOther(c.id);
-    V3<R> ra = rotate(v.Q(a), V3<R>{c.local[0], c.local[1], c.local[2]});
-    V3<R> rb = rotate(v.Q(b), V3<R>{c.localB[0], c.localB[1], c.localB[2]});
-    V3<R> delta = ((v.X(a) + ra) - v.X(b)) - rb;
-    R cz = dot(delta, V3<R>{c.n[0], c.n[1], c.n[2]}) - M.alpha * c.c0;
-    R depth = mx(R(0), -(cz + M.alpha * c.c0));
-    if (c.lambda[2] < R(-1e-5) || depth > R(1e-6))
-      n += 1;
-    depthMax = mx(depthMax, depth);
+  const bool lead = lane == 0, foot = lane < sv.numFeet;
+  const size_t at = size_t(e) * sv.numFeet + lane;
+  R contacts = 0, penetration = 0, off[3] = {0, 0, 0}, mean[3] = {0, 0, 0}, air = 0, touch = 0;
+  if (lead) {
+    if (sv.selfContacts)
+      contacts = sv.selfContacts[e];
+    if (sv.selfPenetration)
+      penetration = sv.selfPenetration[e];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      off[k] = sv.rootOffset[size_t(e) * 3 + k];
+    if (sv.meanVelocity) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        mean[k] = sv.meanVelocity[size_t(e) * 3 + k];
+    }
   }
-  if (sv.selfContacts)
-    sv.selfContacts[e] = maximumNan(sv.selfContacts[e], n);
-  if (sv.selfPenetration)
-    sv.selfPenetration[e] = maximumNan(sv.selfPenetration[e], depthMax);
+  if (foot) {
+    if (sv.airTime)
+      air = sv.airTime[at];
+    if (sv.contactTime)
+      touch = sv.contactTime[at];
+  }
   auto put = [](R *out, size_t i, V3<R> u) {
     if (out) {
       out[3 * i] = u.x;
@@ -246,27 +258,50 @@ __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const Devi
       out[3 * i + 2] = u.z;
     }
   };
-  const Q4<R> q1 = v.Q(1), root = q1 * Q4<R>{sv.rootInv[0], sv.rootInv[1], sv.rootInv[2], sv.rootInv[3]};
-  const V3<R> w1 = v.W(1), v1{s.v[0][1], s.v[1][1], s.v[2][1]};
-  put(sv.gravity, e, rotate(conj(root), V3<R>{0, 0, -1}));
-  put(sv.angularVelocity, e, rotate(conj(root), w1));
-  const R *off = sv.rootOffset + size_t(e) * 3;
-  const V3<R> rootR = -rotate(q1, V3<R>{off[0], off[1], off[2]});
-  const V3<R> origin = v1 + cross(w1, rootR);
-  put(sv.originVelocity, e, origin);
-  put(sv.linearVelocity, e, rotate(conj(root), origin));
-  if (sv.meanVelocity) {
+  if (lead) {
+    R n = 0, depthMax = 0;
+    for (int i = 0; i < s.nsc; ++i) {
+      const auto &c = s.sc[i];
+      int a = scBody(c.id), b = scOther(c.id);
+      V3<R> ra = rotate(v.Q(a), V3<R>{c.local[0], c.local[1], c.local[2]});
+      V3<R> rb = rotate(v.Q(b), V3<R>{c.localB[0], c.localB[1], c.localB[2]});
+      V3<R> delta = ((v.X(a) + ra) - v.X(b)) - rb;
+      R cz = dot(delta, V3<R>{c.n[0], c.n[1], c.n[2]}) - M.alpha * c.c0;
+      R depth = mx(R(0), -(cz + M.alpha * c.c0));
+      if (c.lambda[2] < R(-1e-5) || depth > R(1e-6))
+        n += 1;
+      depthMax = mx(depthMax, depth);
+    }
+    if (sv.selfContacts)
+      sv.selfContacts[e] = maximumNan(contacts, n);
+    if (sv.selfPenetration)
+      sv.selfPenetration[e] = maximumNan(penetration, depthMax);
+    const Q4<R> q1 = v.Q(1), root = q1 * Q4<R>{sv.rootInv[0], sv.rootInv[1], sv.rootInv[2], sv.rootInv[3]};
+    const V3<R> w1 = v.W(1), v1{s.v[0][1], s.v[1][1], s.v[2][1]};
+    put(sv.gravity, e, rotate(conj(root), V3<R>{0, 0, -1}));
+    put(sv.angularVelocity, e, rotate(conj(root), w1));
+    const V3<R> rootR = -rotate(q1, V3<R>{off[0], off[1], off[2]});
+    const V3<R> origin = v1 + cross(w1, rootR);
+    put(sv.originVelocity, e, origin);
+    put(sv.linearVelocity, e, rotate(conj(root), origin));
     // mean_velocity_world.lerp_(origin, alpha) (bam_env.py:343-345) as
     // mean + alpha (origin - mean)
-    R *m = sv.meanVelocity + size_t(e) * 3;
-    m[0] = m[0] + sv.meanAlpha * (origin.x - m[0]);
-    m[1] = m[1] + sv.meanAlpha * (origin.y - m[1]);
-    m[2] = m[2] + sv.meanAlpha * (origin.z - m[2]);
+    put(sv.meanVelocity, e,
+        V3<R>{mean[0] + sv.meanAlpha * (origin.x - mean[0]), mean[1] + sv.meanAlpha * (origin.y - mean[1]),
+              mean[2] + sv.meanAlpha * (origin.z - mean[2])});
   }
-  const R h = M.dt;
-  for (int f = 0; f < sv.numFeet; ++f) {
-    const int body = sv.feet[f];
-    const size_t k = size_t(e) * sv.numFeet + f;
+  if (foot) {
+    // (the arguments selected, not indexed by lane: indexed they would be
+    // copied to scratch memory)
+    int body = sv.feet[0];
+    V3<R> site{sv.sites[0][0], sv.sites[0][1], sv.sites[0][2]};
+#pragma unroll
+    for (int f = 1; f < DUCK_MAX_FEET; ++f) {
+      body = lane == f ? sv.feet[f] : body;
+      site.x = lane == f ? sv.sites[f][0] : site.x;
+      site.y = lane == f ? sv.sites[f][1] : site.y;
+      site.z = lane == f ? sv.sites[f][2] : site.z;
+    }
     V3<R> force{0, 0, 0};
     for (int i = 0; i < s.ngc; ++i) {
       const auto &c = s.gc[i];
@@ -278,16 +313,17 @@ __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const Devi
       force.y += g.y;
       force.z += g.z;
     }
-    put(sv.footForces, k, force);
-    const V3<R> r = rotate(v.Q(body), V3<R>{sv.sites[f][0], sv.sites[f][1], sv.sites[f][2]});
+    put(sv.footForces, at, force);
+    const V3<R> r = rotate(v.Q(body), site);
     const V3<R> vb{s.v[0][body], s.v[1][body], s.v[2][body]};
-    put(sv.sitePositions, k, v.X(body) + r);
-    put(sv.siteVelocities, k, vb + cross(v.W(body), r));
+    put(sv.sitePositions, at, v.X(body) + r);
+    put(sv.siteVelocities, at, vb + cross(v.W(body), r));
     const bool contact = norm(force) > R(1e-5);
+    const R h = M.dt;
     if (sv.airTime)
-      sv.airTime[k] = contact ? R(0) : sv.airTime[k] + h;
+      sv.airTime[at] = contact ? R(0) : air + h;
     if (sv.contactTime)
-      sv.contactTime[k] = contact ? sv.contactTime[k] + h : R(0);
+      sv.contactTime[at] = contact ? touch + h : R(0);
   }
 }
 

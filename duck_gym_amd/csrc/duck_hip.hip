@@ -263,7 +263,7 @@ struct BatchBase {
   virtual void taskLog(const DuckTask &, const unsigned char *, const void *, const void *,
                        const void *, double, void *, hipStream_t) = 0;
   virtual void servo(const DuckServo &, const ServoBuffers &, hipStream_t) = 0;
-  virtual void servoSubstep(const DuckServo &, const DuckServoSubstep &, hipStream_t) = 0;
+  virtual void servoSubsteps(const DuckServo &, const DuckServoSubstep &, int, hipStream_t) = 0;
   virtual void kernelInfo(int which, long long *out) = 0;
 };
 
@@ -622,7 +622,7 @@ public:
     taskLogReduceKernel<R><<<1, 64, 0, s>>>(rows, count, static_cast<R *>(out));
     launched("taskLogReduceKernel");
   }
-  void servoSubstep(const DuckServo &p, const DuckServoSubstep &io, hipStream_t s) override {
+  void servoSubsteps(const DuckServo &p, const DuckServoSubstep &io, int substeps, hipStream_t s) override {
     DeviceGuard guard(device);
     const int nb = host.bodies.size();
     require(nb >= 2, "servo substep: the model needs a root body (body 1)");
@@ -665,7 +665,7 @@ public:
             "servo substep: mean_velocity_alpha outside [0, 1]");
     sv.meanAlpha = R(io.mean_velocity_alpha);
     StepArgs args{dModel, dFrames, dPoints, dStates, blobBytes, count, nullptr, nullptr, nullptr,
-                  1, kMotorControls, 0, 0,
+                  substeps, kMotorControls, 0, 0,
                   nb, int(host.joints.size()), int(host.shapes.size()), int(host.pairs.size()),
                   customBodies ? 1 : 0, perWave(count)};
     const int blocks = (count + args.perWave - 1) / args.perWave;
@@ -1252,8 +1252,13 @@ int duck_servo(void *handle, const DuckServo *servo, const void *target, void *h
 }
 int duck_servo_substep(void *handle, const DuckServo *servo, const DuckServoSubstep *io,
                        void *hip_stream) {
+  return duck_servo_substeps(handle, servo, io, 1, hip_stream);
+}
+int duck_servo_substeps(void *handle, const DuckServo *servo, const DuckServoSubstep *io, int substeps,
+                        void *hip_stream) {
   return guarded([&] {
     auto *b = as(handle);
+    require(substeps >= 1, "servo: substeps below one");
     require(servo != nullptr && io != nullptr, "null servo parameters");
     require(io->target && io->history && io->initialized && io->root_offset &&
                 io->previous_motor && io->previous_applied,
@@ -1266,7 +1271,7 @@ int duck_servo_substep(void *handle, const DuckServo *servo, const DuckServoSubs
       require(std::isfinite(v), "servo: non-finite parameter");
     require(servo->resistance != 0 && servo->dtheta_stribeck != 0 && servo->vin_min > 0,
             "servo: resistance, dtheta_stribeck and vin_min must be nonzero");
-    b->servoSubstep(*servo, *io, st(hip_stream));
+    b->servoSubsteps(*servo, *io, substeps, st(hip_stream));
   });
 }
 int duck_reference(void *handle, const void *target, const void *force, int substeps, double kp,

@@ -68,6 +68,8 @@ def library():
             "duck_servo": (ip, [vp, ctypes.POINTER(DuckServo), vp, vp, ip] + [vp] * 7),
             "duck_servo_substep": (ip, [vp, ctypes.POINTER(DuckServo),
                                         ctypes.POINTER(DuckServoSubstep), vp]),
+            "duck_servo_substeps": (ip, [vp, ctypes.POINTER(DuckServo),
+                                        ctypes.POINTER(DuckServoSubstep), ip, vp]),
         }
         for name, (res, args) in sig.items():
             fn = getattr(lib, name)
@@ -86,7 +88,7 @@ EXPORTED = (
     "duck_export_state",
     "duck_import_state", "duck_last_error", "duck_task_obs_dim", "duck_task_targets",
     "duck_task_step", "duck_task_observe", "duck_task_log", "duck_task_reset_inputs", "duck_servo",
-    "duck_servo_substep",
+    "duck_servo_substep", "duck_servo_substeps",
     "duck_sequential_step",
 )
 
@@ -417,9 +419,8 @@ class CudaBatch:
         mean-velocity filter mean += alpha (origin velocity - mean)
         (bam_env.py:343-345), in one launch.  Outputs are written into the
         tensors given (any may be None); in/out tensors are updated in place.
-        `count` of them run with the same buffers, the history's cursor moving
-        on by one slot each; the buffers are looked over once (some 20 tensors:
-        as long on the host as a substep of 4096 environments on the GPU)."""
+        `count` of them run in one launch with the same buffers, the history's
+        cursor moving on by one slot each."""
         E, J = self.num_envs, self.num_joints
         F = len(feet)
         if F > MAX_FEET:
@@ -428,6 +429,7 @@ class CudaBatch:
         stream = torch.cuda.current_stream(self.device)
         io.target = self._check(target, [E, J], None, stream).value
         io.history = self._check(history, [slots, E, J], None, stream).value
+        io.cursor = int(cursor)
         io.initialized = self._check(initialized, [E], torch.bool, stream).value
         io.root_offset = self._check(root_offset, [E, 3], None, stream).value
         io.previous_motor = self._check(previous_motor, [E, J], None, stream).value
@@ -455,13 +457,11 @@ class CudaBatch:
             io.foot_bodies[f] = int(feet[f])
             for k in range(3):
                 io.foot_sites[f][k] = float(sites[f][k])
-        launch, raw = library().duck_servo_substep, ctypes.c_void_p(stream.cuda_stream)
         with torch.cuda.device(self.device):
-            for k in range(count):
-                io.cursor = int(cursor) if k == 0 else (int(cursor) + k) % slots
-                code = launch(self._h, ctypes.byref(params), ctypes.byref(io), raw)
-                if code:
-                    _raise(code, "servo_substep")
+            code = library().duck_servo_substeps(self._h, ctypes.byref(params), ctypes.byref(io),
+                                                 int(count), ctypes.c_void_p(stream.cuda_stream))
+        if code:
+            _raise(code, "servo_substep")
 
     def task_obs_dim(self, task):
         return int(library().duck_task_obs_dim(ctypes.byref(task), self.num_joints))

@@ -84,7 +84,8 @@ class ServoLoop:
     world velocity every substep (bam_env.py:343-345, weight
     -expm1(-dt / tau)); `reset` clears it.
 
-    `fused` (default) runs a substep as one launch (`CudaBatch.servo_substep`);
+    `fused` (default) runs the substeps as one launch, or one each where a
+    callback comes between them (`CudaBatch.servo_substep`);
     otherwise as the reference loop does: the servo kernel, the motor step,
     the self-contact query and the refresh arithmetic in torch.  The root
     frame is body 1's frame times the conjugate of `root_principal_quat`
@@ -183,14 +184,14 @@ class ServoLoop:
         The callback sees the state and refresh quantities of each substep.
         The unfused path calls it where the reference does, before the
         self-contact maxima, the mean-velocity filter and the timers take
-        this substep in; in the fused path, one launch per substep, they
+        this substep in; in the fused path they
         already include it when the callback runs."""
         target = target.contiguous()
         self.self_contacts.zero_()
         self.self_penetration.zero_()
         if self.fused:
             # without a callback nothing can change between the substeps: one
-            # call for all of them
+            # launch for all of them
             each = 1 if substep_callback is not None else count
             for _ in range(0, count, max(each, 1)):
                 self.batch.servo_substep(

@@ -327,6 +327,11 @@ typedef struct DuckServoSubstep {
  * replaces the reference loop's five calls and torch arithmetic. */
 int duck_servo_substep(void *handle, const DuckServo *servo, const DuckServoSubstep *io,
                        void *hip_stream);
+/* `substeps` (>= 1) of them in one launch, with the same buffers and the
+ * cursor moving on by one slot each: the results of as many calls of
+ * duck_servo_substep.  The caller advances `cursor` by `substeps`. */
+int duck_servo_substeps(void *handle, const DuckServo *servo, const DuckServoSubstep *io, int substeps,
+                        void *hip_stream);
 
 /* ---- Explicit-sequential step (src/solver.cpp:315-537) ----
  * The step of the reference's independent float64 solver, duck::Solver::step

@@ -83,3 +83,48 @@ def test_servo_substeps_are_the_same_however_many_share_a_wave(lag, fp64):
                 x.history.transpose(0, 1), x.gravity, x.lin_vel, x.contact_force, x.site_pos,
                 x.air_time, x.contact_time, x.self_contacts, x.self_penetration,
                 x.mean_velocity) for x in loops])
+
+
+@pytest.mark.parametrize("lag,fp64", [(0, False), (1, False), (2, True), (6, False)])
+def test_servo_substeps_of_one_launch_are_those_of_a_launch_each(lag, fp64):
+    """Histories fresh and filled, a reset between, an environment whose
+    target is refused (its step fails, its servo goes on), lags below and
+    above the substeps of a launch."""
+    text, meta = model_text(self_contact=True)
+    dtype, E = (torch.float64 if fp64 else torch.float32), 37
+    home, rng = np.array(meta["home"]), np.random.default_rng(5)
+    feet = [meta["body_names"].index(n) for n in ("left_foot", "right_foot")]
+    t = lambda a: torch.tensor(a, dtype=dtype, device=DEV)  # noqa: E731
+    every = torch.ones(E, dtype=torch.bool, device=DEV)
+    loops = []
+    for _ in range(2):
+        b = CudaBatch.from_text(text, E, DT, ITER, 0, fp64)
+        b.reset(every, t(np.tile(home, (E, 1))), t(np.zeros((E, 6))))
+        loops.append(ServoLoop(b, servo_params(**SYNTHETIC_SUPPLY, lag=lag), home, [0.0, 0.0, 0.01],
+                               root_principal_quat=meta["root_iquat"], feet=feet,
+                               foot_sites=[[0.01, 0.0, -0.006]] * 2, mean_velocity_tau=0.2))
+    some = torch.arange(E, device=DEV) % 5 == 2
+    seen = []
+    for k, count in enumerate((4, 1, 5, 3, 4)):
+        targets = home + rng.uniform(-0.3, 0.3, (E, 14))
+        if k == 2:
+            targets[8, 3] = np.nan
+        loops[0].substeps(t(targets), count)
+        loops[1].substeps(t(targets), count, substep_callback=lambda loop: seen.append(loop.cursor))
+        if k == 3:
+            for loop in loops:
+                loop.reset(some)
+                loop.batch.reset(some, t(np.tile(home, (E, 1))), t(np.zeros((E, 6))))
+        a, b = ([*x.batch.state(), x.motor, x.previous_motor, x.previous_applied, x.initialized, x.history,
+                 x.gravity, x.ang_vel, x.lin_vel, x.origin_velocity, x.contact_force, x.site_pos, x.site_vel,
+                 x.air_time, x.contact_time, x.self_contacts, x.self_penetration, x.mean_velocity]
+                for x in loops)
+        for i, (p, q) in enumerate(zip(a, b)):
+            assert torch.equal(p.nan_to_num(-9.0) if p.is_floating_point() else p,
+                               q.nan_to_num(-9.0) if q.is_floating_point() else q), (k, i)
+        assert loops[0].cursor == loops[1].cursor
+        raw = [x.batch.export_state().cpu().numpy() for x in loops]
+        codec = loops[0].batch.codec()
+        header = codec.L["gc"]
+        assert np.array_equal(raw[0][:, :header], raw[1][:, :header]), k
+    assert len(seen) == 17 and loops[0].batch.state()[2][:, 5].sum() == 1
