@@ -308,16 +308,19 @@ class Batch final : public BatchBase {
   // Environments a wave of the full step advances in a launch of n.  The
   // environments of a wave take each other's turns (contact rounds, body-pair
   // queries, third colours, the double step's angle branches), so they get
-  // waves of their own while those are free.  Float waves that share a CU cost
-  // each other more than that (500 standing environments as 500, 250 and 125
-  // waves: 94.5, 90.8, 90.1 us; a sweep of 100 as 100, 50 and 25: 135, 139,
-  // 143 us), so they stop at one to a CU; in double the turns cost more (501
-  // environments as 501, 251 and 126 waves: 298, 323, 343 us), so those stop
-  // where every wave is still resident.
-  static constexpr int kResident =
+  // waves of their own while the launch stays within a quarter of the waves
+  // that the device holds at once: a process has four hardware queues, so the
+  // launches of as many streams still run side by side.  Past that line they
+  // take turns, which costs more than the own waves give one launch alone
+  // (MicroDuck in double, us per step: two batches of 500 as 125 waves each
+  // 323, as 500 waves 568; three of 250 as 125 waves 303, as 250 waves 433;
+  // alone, 500 as 125, 250 and 500 waves 338, 319 and 296).  For float that
+  // quarter is one wave per compute unit, where waves begin to cost each other
+  // LDS turns anyway (a sweep of 100 as 100, 50 and 25 waves: 135, 139, 143).
+  static constexpr int kResident = // workgroups of a compute unit's LDS
       int(160 * 1024 / (sizeof(Frames<R, B, J>) + G * sizeof(typename Stepper<R, B, J, CG, CS, L, PL>::Env)));
   int perWave(int n) const {
-    const int waves = cus * (sizeof(R) == sizeof(float) ? 1 : kResident);
+    const int waves = cus * kResident / 4;
     int per = 1;
     while (per < G && (n + per - 1) / per > waves)
       per *= 2;

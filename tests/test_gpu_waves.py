@@ -10,6 +10,7 @@ import torch
 from duck_gym_amd import CudaBatch
 from duck_gym_amd.microduck import model_text
 from duck_gym_amd.servo import SYNTHETIC_SUPPLY, ServoLoop, servo_params
+from model_text import caterpillar
 
 pytestmark = pytest.mark.gpu
 
@@ -20,9 +21,29 @@ def _parts(fp64):
     """A batch of four environments to a wave (the last one holding three),
     and the same environments as two to a wave (the last one alone), one to a
     wave, and three in all."""
-    waves = torch.cuda.get_device_properties(0).multi_processor_count * (2 if fp64 else 1)
+    # own waves up to a quarter of those that fit: a float workgroup takes a
+    # quarter of a compute unit, a double one half
+    waves = torch.cuda.get_device_properties(0).multi_processor_count // (2 if fp64 else 1)
     return [slice(0, 2 * waves + 3), slice(0, waves + 1), slice(waves + 1, 2 * waves),
             slice(2 * waves, 2 * waves + 3)]
+
+
+@pytest.mark.parametrize("fp64,split,large", [(False, False, False), (True, False, False), (True, True, False),
+                                              (False, False, True), (True, False, True), (True, True, True)])
+def test_launches_of_four_streams_fit_the_device_together(fp64, split, large):
+    """Environments get waves of their own only while four such launches stay
+    resident together; past that a wave is filled."""
+    text = caterpillar(20, pairs=False) if large else model_text()[0]
+    room = None
+    for n in (4096, 1, 63, 64, 65, 100, 128, 129, 192, 193, 250, 256, 257, 500, 513, 1000, 1025):
+        info = CudaBatch.from_text(text, n, DT, ITER, 0, fp64, split_solve=split).kernel_info()
+        if room is None:
+            cus = torch.cuda.get_device_properties(0).multi_processor_count
+            room, most = cus * info["workgroups_per_cu"], info["envs_per_workgroup"]
+            assert most == (2 if large else 4)
+        assert info["envs_per_workgroup"] == most or 4 * info["workgroups_per_launch"] <= room, n
+        if 4 * n <= room:
+            assert info["envs_per_workgroup"] == 1, n
 
 
 def _batches(pairs, fp64):
