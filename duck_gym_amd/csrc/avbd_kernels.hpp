@@ -726,7 +726,10 @@ __global__ void framesKernel(const DeviceModel<R> *model, Frames<R, B, J> *out) 
 // hold what no other field gives and the first kDenseContacts ground contacts
 // (DenseEnv); further contacts stay in the blob.  The operations are the full
 // step's in its order: bitwise the same states.
-template <class R, int B, int J, int CG, int CS, int L, int PL, bool Servo, bool Pairs, bool Dense = false>
+// Many: a launch of several servo substeps (a build of its own: the loop around
+// prologue, controls and epilogue costs the registers of one substep).
+template <class R, int B, int J, int CG, int CS, int L, int PL, bool Servo, bool Pairs, bool Dense = false,
+          bool Many = false>
 __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R> &sv, int block) {
   static_assert(!Dense || (!Servo && !Pairs && sizeof(R) == sizeof(float) && L == 16 && B <= L && J <= L &&
                            kDenseContacts <= CG),
@@ -772,7 +775,11 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   const int here = args.count - e0 < per ? args.count - e0 : per;
   const bool own = g < here;
   const int e = Fill && !own ? e0 : e0 + g;
-  const bool valid = Fill || own;
+  // (Always true where groups repeat.  Whether the compiler may know it moves
+  // its schedule and its spills; it is told where that measured faster: not in
+  // the MicroDuck-sized servo, 110.8 -> 105.9 us per substep of four at 4096.)
+  constexpr bool Known = Fill && !(Servo && L == 16);
+  const bool valid = Known || e < args.count;
   Env *envs = envsOf + wave * G;
   Env &E = envs[g];
   // (a model without body pairs: none of their code is compiled)
@@ -880,8 +887,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
       massPattern |= (E.s.mass[b] > 0) != (F.mass[b] > 0);
   const bool defaultSchedule = groupOr<L>(massPattern) == 0;
   // ---- controls (extension.cu:87-110 / kernel.cuh:448-466) ----
-  // (once per launch; in a servo launch before every substep, with the
-  // channels its prologue forms)
+  // (once per launch; with Many before every substep, with the channels its
+  // prologue forms)
   bool active = false, ran = false;
   // What the blob's drive parameters and colouring hold before this launch
   // (read before any lane rewrites the stamps).
@@ -993,7 +1000,9 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   }
   meet();
   };
-  if constexpr (!Servo)
+  if constexpr (Servo && !Many)
+    servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, own, args.count, 0, servoIn, ctl);
+  if constexpr (!Many)
     setControls();
 
   Step stp{M, points, F, E, lane, {}};
@@ -1015,25 +1024,26 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   const int slot = P == 1 ? lane : (lane & 7) + 8 * (lane / (8 * P));
   const R h = M.dt, alpha = M.alpha, gamma = M.gamma, ag = alpha * gamma;
 
-  // (a servo launch ends every substep, also one that no environment steps,
-  // at the top of the next round; it writes back as many contacts as any of
-  // its substeps had, as a launch each would have)
+  // (a launch of many servo substeps ends each of them, also one that no
+  // environment steps, at the top of the next round; it writes back as many
+  // contacts as any of its substeps had, as a launch each would have)
   int mostGround = 0, mostSelf = 0;
-  for (int sub = 0; sub < args.substeps + (Servo ? 1 : 0); ++sub) {
-    if constexpr (Servo) {
+  const int substeps = Servo && !Many ? 1 : args.substeps;
+  for (int sub = 0; sub < substeps + (Many ? 1 : 0); ++sub) {
+    if constexpr (Many) {
       if (sub > 0 && own) {
         servoEpilogue<R, B, J, CG, CS, L>(sv, M, E, e, lane);
         mostGround = mostGround > E.s.ngc ? mostGround : E.s.ngc;
         mostSelf = mostSelf > E.s.nsc ? mostSelf : E.s.nsc;
       }
       __syncthreads();
-      if (sub == args.substeps)
+      if (sub == substeps)
         break;
       servoPrologue<R, B, J, CG, CS, L>(sv, M, F, E, e, lane, own, args.count, sub, servoIn, ctl);
       setControls();
     }
     if (!__any(active)) {
-      if constexpr (Servo)
+      if constexpr (Many)
         continue;
       else
         break;
@@ -1958,6 +1968,9 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
     meet();
     meet();
   }
+  if constexpr (Servo && !Many)
+    if (own)
+      servoEpilogue<R, B, J, CG, CS, L>(sv, M, E, e, lane);
   // The colouring of an environment that stepped is the model's exactly when
   // no body took a fresh colour; it is written when the blob holds another.
   const int plan = valid ? E.writeback : 0;
@@ -1985,8 +1998,8 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
         gs->colors[lane] = lane < nb ? M.colors[lane] : 0;
     }
   } else if (own) {
-    storeEnv<State>(gs, E.s, lane, L, plan >> 8, (plan >> 1) & 3, writeColours, Servo ? mostGround : E.s.ngc,
-                    Servo ? mostSelf : E.s.nsc);
+    storeEnv<State>(gs, E.s, lane, L, plan >> 8, (plan >> 1) & 3, writeColours, Many ? mostGround : E.s.ngc,
+                    Many ? mostSelf : E.s.nsc);
   }
 }
 
@@ -2016,19 +2029,20 @@ __global__ __launch_bounds__(64 * kDenseWaves, 2) __attribute__((aligned(32768))
       args, none, xcdBlock(blockIdx.x, gridDim.x) * kDenseWaves + int(threadIdx.x / 64));
 }
 
-// Servo substeps (bam_env.py:307-337 with refresh()), on a 32 KiB boundary
+// A servo substep (bam_env.py:307-337 with refresh()), on a 32 KiB boundary
 // like advanceKernel.  Bound, as the step, by the dependent chains of the
 // slowest wave; what the servo adds waits for memory, so its buffers are read
-// with the controls, ahead of the staging, and the substeps of a control step
-// run in one launch (no staging and write-back between them, and a wave that
-// is slow in one substep holds up no other before the last).  A control step
-// of four substeps and a state, 4096 environments: 534 -> 527 us with a launch
-// each before, 662 -> 647 us where some robots have fallen; a launch each with
-// the buffers read where they were used 690 us there.
-template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true>
+// with the controls, ahead of the staging.  One substep of the biped with body
+// pairs, a launch each: 117.8 us at 4096 environments, 322 us at 12288 (133.9
+// and 367 us when one substep ran the loop of many).
+// Many: all substeps of a control step in one launch (no staging and
+// write-back between them, and a wave that is slow in one substep holds up no
+// other before the last): four of them 105.9 us each at 4096.
+template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L), bool Pairs = true,
+          bool Many = false>
 __global__ __launch_bounds__(64) __attribute__((aligned(32768))) void servoStepKernel(StepArgs args,
                                                                                    ServoArgs<R> servo) {
-  stepBody<R, B, J, CG, CS, L, PL, true, Pairs>(args, servo, xcdBlock(blockIdx.x, gridDim.x));
+  stepBody<R, B, J, CG, CS, L, PL, true, Pairs, false, Many>(args, servo, xcdBlock(blockIdx.x, gridDim.x));
 }
 
 } // namespace duckhip

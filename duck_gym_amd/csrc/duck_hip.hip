@@ -327,6 +327,30 @@ class Batch final : public BatchBase {
     return per;
   }
 
+  // The servo substep's kernel; `many`: the build for several in one launch.
+  // Float has one (4096 biped environments, us per substep: four in one launch
+  // 105.9 with body pairs and 98.3 without, four launches 114.0 and 107.5).  In
+  // double its loop holds 0.8 to 1.7 KB of spills per lane and is no faster
+  // (647 and 612 against 631 and 601; 700 of a 24-segment chain 862 against
+  // 848), so a double batch launches the one-substep build each time.
+  static constexpr bool kManySubsteps = sizeof(R) == sizeof(float);
+  using ServoKernel = void (*)(StepArgs, ServoArgs<R>);
+  ServoKernel servoKernelOf(bool many) const {
+    const bool pairless = kPairless && host.pairs.empty();
+    if constexpr (kManySubsteps) {
+      if (many) {
+        if constexpr (kPairless)
+          if (pairless)
+            return &servoStepKernel<R, B, J, CG, CS, L, PL, false, true>;
+        return &servoStepKernel<R, B, J, CG, CS, L, PL, true, true>;
+      }
+    }
+    if constexpr (kPairless)
+      if (pairless)
+        return &servoStepKernel<R, B, J, CG, CS, L, PL, false>;
+    return &servoStepKernel<R, B, J, CG, CS, L, PL>;
+  }
+
   void advance(unsigned char *states, int n, const void *targets, const void *forces,
                const void *motor, int substeps, double kp, double limit, hipStream_t s,
                int mode = -1) {
@@ -672,16 +696,14 @@ public:
                   nb, int(host.joints.size()), int(host.shapes.size()), int(host.pairs.size()),
                   customBodies ? 1 : 0, perWave(count)};
     const int blocks = (count + args.perWave - 1) / args.perWave;
+    const bool many = kManySubsteps && substeps > 1;
+    const auto kernel = servoKernelOf(many);
     wait(s);
-    if constexpr (kPairless) {
-      if (host.pairs.empty())
-        servoStepKernel<R, B, J, CG, CS, L, PL, false><<<blocks, 64, 0, s>>>(args, sv);
-      else
-        servoStepKernel<R, B, J, CG, CS, L, PL><<<blocks, 64, 0, s>>>(args, sv);
-    } else {
-      servoStepKernel<R, B, J, CG, CS, L, PL><<<blocks, 64, 0, s>>>(args, sv);
+    for (int launch = 0; launch < (many ? 1 : substeps); ++launch) {
+      sv.cursor = (io.cursor + launch) % (p.lag + 1);
+      kernel<<<blocks, 64, 0, s>>>(args, sv);
+      launched("servoStepKernel");
     }
-    launched("servoStepKernel");
     record(s);
   }
   void servo(const DuckServo &p, const ServoBuffers &io, hipStream_t s) override {
@@ -693,29 +715,27 @@ public:
     record(s);
   }
   void layout(long long *out) const override;
-  // Resources of the kernel this batch's duck_step (which = DUCK_KERNEL_STEP)
-  // or duck_servo_substep (DUCK_KERNEL_SERVO_SUBSTEP) launches -- the dense
-  // step, or the build without body-pair code for a model without pairs: VGPRs, static LDS and
+  // Resources of the kernel this batch's duck_step (which = DUCK_KERNEL_STEP),
+  // duck_servo_substep (DUCK_KERNEL_SERVO_SUBSTEP) or duck_servo_substeps of
+  // several (DUCK_KERNEL_SERVO_SUBSTEPS) launches -- the dense step, or the
+  // build without body-pair code for a model without pairs: VGPRs, static LDS and
   // scratch per lane from the code object, resident workgroups per CU from
   // the runtime's occupancy calculator, lanes and environments per
   // workgroup, and workgroups per launch.
   void kernelInfo(int which, long long *out) override {
     DeviceGuard guard(device);
-    require(which == DUCK_KERNEL_STEP || which == DUCK_KERNEL_SERVO_SUBSTEP,
+    require(which == DUCK_KERNEL_STEP || which == DUCK_KERNEL_SERVO_SUBSTEP ||
+                which == DUCK_KERNEL_SERVO_SUBSTEPS,
             "kernel_info: unknown kernel");
-    const bool pairless = kPairless && host.pairs.empty();
     const void *fn = nullptr;
     int waves = 1; // of a workgroup
     if (which == DUCK_KERNEL_STEP)
       fn = reinterpret_cast<const void *>(&advanceKernel<R, B, J, CG, CS, L, PL>);
     else
-      fn = reinterpret_cast<const void *>(&servoStepKernel<R, B, J, CG, CS, L, PL>);
-    if constexpr (kPairless) {
-      if (pairless && which == DUCK_KERNEL_STEP)
+      fn = reinterpret_cast<const void *>(servoKernelOf(kManySubsteps && which == DUCK_KERNEL_SERVO_SUBSTEPS));
+    if constexpr (kPairless)
+      if (host.pairs.empty() && which == DUCK_KERNEL_STEP)
         fn = reinterpret_cast<const void *>(&advanceKernel<R, B, J, CG, CS, L, PL, false>);
-      if (pairless && which == DUCK_KERNEL_SERVO_SUBSTEP)
-        fn = reinterpret_cast<const void *>(&servoStepKernel<R, B, J, CG, CS, L, PL, false>);
-    }
     if constexpr (kDense) {
       if (which == DUCK_KERNEL_STEP && dense((count + G - 1) / G, kTargetControls)) {
         fn = reinterpret_cast<const void *>(&denseKernel<R, B, J, CG, CS, L, PL>);

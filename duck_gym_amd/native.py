@@ -238,12 +238,13 @@ class CudaBatch:
         return int(library().duck_state_bytes(self._h))
 
     def kernel_info(self, kernel="step"):
-        """Resources of the kernel `step` ("step") or `servo_substep`
-        ("servo_substep") launches (duck_kernel_info): VGPRs, static LDS bytes
+        """Resources of the kernel that `step` ("step"), `servo_substep`
+        ("servo_substep") or `servo_substep` with a count above one
+        ("servo_substeps") launches (duck_kernel_info): VGPRs, static LDS bytes
         per workgroup, scratch bytes per lane, resident workgroups per CU,
         lanes and environments per workgroup, workgroups per launch, and the
         waves per SIMD they give."""
-        which = {"step": 0, "servo_substep": 1}[kernel]
+        which = {"step": 0, "servo_substep": 1, "servo_substeps": 2}[kernel]
         out = (ctypes.c_longlong * 7)()
         code = library().duck_kernel_info(self._h, which, out)
         if code:
@@ -419,8 +420,8 @@ class CudaBatch:
         mean-velocity filter mean += alpha (origin velocity - mean)
         (bam_env.py:343-345), in one launch.  Outputs are written into the
         tensors given (any may be None); in/out tensors are updated in place.
-        `count` of them run in one launch with the same buffers, the history's
-        cursor moving on by one slot each."""
+        `count` of them run with the same buffers (in float32 in one launch),
+        the history's cursor moving on by one slot each."""
         E, J = self.num_envs, self.num_joints
         F = len(feet)
         if F > MAX_FEET:

@@ -84,8 +84,9 @@ class ServoLoop:
     world velocity every substep (bam_env.py:343-345, weight
     -expm1(-dt / tau)); `reset` clears it.
 
-    `fused` (default) runs the substeps as one launch, or one each where a
-    callback comes between them (`CudaBatch.servo_substep`);
+    `fused` (default) runs the substeps as one launch (float32), or one each
+    in float64 and where a callback comes between them
+    (`CudaBatch.servo_substep`);
     otherwise as the reference loop does: the servo kernel, the motor step,
     the self-contact query and the refresh arithmetic in torch.  The root
     frame is body 1's frame times the conjugate of `root_principal_quat`
@@ -191,7 +192,7 @@ class ServoLoop:
         self.self_penetration.zero_()
         if self.fused:
             # without a callback nothing can change between the substeps: one
-            # launch for all of them
+            # call for all of them
             each = 1 if substep_callback is not None else count
             for _ in range(0, count, max(each, 1)):
                 self.batch.servo_substep(

@@ -127,14 +127,15 @@ int duck_reference(void *handle, const void *target, const void *force, int subs
 int duck_reference_noalloc(void *handle, const void *target, const void *force, int substeps,
                            double kp, double limit, void *bodies, void *joints, void *diag);
 
-/* Resources of the kernel that duck_step (which = DUCK_KERNEL_STEP) or
- * duck_servo_substep (DUCK_KERNEL_SERVO_SUBSTEP) launches for this batch (no
+/* Resources of the kernel that duck_step (which = DUCK_KERNEL_STEP),
+ * duck_servo_substep (DUCK_KERNEL_SERVO_SUBSTEP) or duck_servo_substeps of more
+ * than one (DUCK_KERNEL_SERVO_SUBSTEPS) launches for this batch (no
  * reference counterpart: for measurement).  out[7] = VGPRs per lane, static
  * LDS bytes per workgroup, scratch bytes per lane, resident workgroups per CU
  * (the runtime's occupancy calculator), lanes per workgroup, environments per
  * workgroup, workgroups per launch.  Waves per SIMD = workgroups per CU x
  * lanes per workgroup / 64 / 4. */
-enum { DUCK_KERNEL_STEP = 0, DUCK_KERNEL_SERVO_SUBSTEP = 1 };
+enum { DUCK_KERNEL_STEP = 0, DUCK_KERNEL_SERVO_SUBSTEP = 1, DUCK_KERNEL_SERVO_SUBSTEPS = 2 };
 int duck_kernel_info(void *handle, int which, long long *out);
 
 /* Size in bytes of one environment's HBM state blob. */
@@ -327,8 +328,8 @@ typedef struct DuckServoSubstep {
  * replaces the reference loop's five calls and torch arithmetic. */
 int duck_servo_substep(void *handle, const DuckServo *servo, const DuckServoSubstep *io,
                        void *hip_stream);
-/* `substeps` (>= 1) of them in one launch, with the same buffers and the
- * cursor moving on by one slot each: the results of as many calls of
+/* `substeps` (>= 1) of them (float: in one launch) with the same buffers and
+ * the cursor moving on by one slot each: the results of as many calls of
  * duck_servo_substep.  The caller advances `cursor` by `substeps`. */
 int duck_servo_substeps(void *handle, const DuckServo *servo, const DuckServoSubstep *io, int substeps,
                         void *hip_stream);

@@ -106,6 +106,17 @@ def test_servo_substeps_are_the_same_however_many_share_a_wave(lag, fp64):
                 x.mean_velocity) for x in loops])
 
 
+@pytest.mark.parametrize("pairs,fp64,most", [(False, False, 0), (True, False, 48), (False, True, 0), (True, True, 320)])
+def test_one_servo_substep_has_a_build_without_spills(pairs, fp64, most):
+    """A single substep (duck_servo_substep, a loop with a callback) does not
+    run the loop over substeps, whose spills reach 496 bytes per lane; what
+    scratch memory is left holds the body-pair geometry (float: 48 bytes)."""
+    b = CudaBatch.from_text(model_text(self_contact=pairs)[0], 5, DT, ITER, 0, fp64)
+    one, many = b.kernel_info("servo_substep"), b.kernel_info("servo_substeps")
+    assert one["scratch_bytes_per_lane"] <= most
+    assert one == many if fp64 else one["vgprs"] < many["vgprs"]
+
+
 @pytest.mark.parametrize("lag,fp64", [(0, False), (1, False), (2, True), (6, False)])
 def test_servo_substeps_of_one_launch_are_those_of_a_launch_each(lag, fp64):
     """Histories fresh and filled, a reset between, an environment whose
