@@ -776,9 +776,12 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   const bool own = g < here;
   const int e = Fill && !own ? e0 : e0 + g;
   // (Always true where groups repeat.  Whether the compiler may know it moves
-  // its schedule and its spills; it is told where that measured faster: not in
-  // the MicroDuck-sized servo, 110.8 -> 105.9 us per substep of four at 4096.)
-  constexpr bool Known = Fill && !(Servo && L == 16);
+  // its schedule and its spills; it is told where that measured faster: in the
+  // float step with body pairs (4096 environments, us: 96.8 told, 98.9 not) and
+  // the generic state (2048 float chains of 24: 410, 423); not in the
+  // MicroDuck-sized servo (a substep of four: 110.8, 105.9), the step without
+  // pairs (eight substeps: 625, 621.5) and double (split solve: 486, 480).)
+  constexpr bool Known = Fill && (L != 16 || (!Servo && Pairs && sizeof(R) == sizeof(float)));
   const bool valid = Known || e < args.count;
   Env *envs = envsOf + wave * G;
   Env &E = envs[g];
