@@ -21,6 +21,7 @@ physically plausible set for tests and benchmarks -- not BAM's fitted values.
 from __future__ import annotations
 
 import math
+import operator
 
 import torch
 
@@ -187,6 +188,7 @@ class ServoLoop:
         self-contact maxima, the mean-velocity filter and the timers take
         this substep in; in the fused path they
         already include it when the callback runs."""
+        count = operator.index(count)
         target = target.contiguous()
         self.self_contacts.zero_()
         self.self_penetration.zero_()
