@@ -772,15 +772,17 @@ __device__ __forceinline__ void stepBody(const StepArgs &args, const ServoArgs<R
   // environments to a wave; one environment, four steps: 337 -> 309 us).
   const int per = Dense ? G : args.perWave, e0 = block * per;
   constexpr bool Fill = !Dense;
+  static_assert(!Fill || W == 1, "a repeated group reads its environment before the same wave writes it");
   const int here = args.count - e0 < per ? args.count - e0 : per;
   const bool own = g < here;
   const int e = Fill && !own ? e0 : e0 + g;
   // (Always true where groups repeat.  Whether the compiler may know it moves
   // its schedule and its spills; it is told where that measured faster: in the
   // float step with body pairs (4096 environments, us: 96.8 told, 98.9 not) and
-  // the generic state (2048 float chains of 24: 410, 423); not in the
-  // MicroDuck-sized servo (a substep of four: 110.8, 105.9), the step without
-  // pairs (eight substeps: 625, 621.5) and double (split solve: 486, 480).)
+  // the generic state (a servo substep of 700 chains of 24 in float: 276, 278,
+  // in double: 854, 859); not in the MicroDuck-sized servo (a substep of four:
+  // 110.8, 105.9), the step without pairs (eight substeps: 625, 621.5) and
+  // double (split solve: 486, 480).)
   constexpr bool Known = Fill && (L != 16 || (!Servo && Pairs && sizeof(R) == sizeof(float)));
   const bool valid = Known || e < args.count;
   Env *envs = envsOf + wave * G;
