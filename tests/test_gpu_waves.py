@@ -160,3 +160,48 @@ def test_servo_substeps_of_one_launch_are_those_of_a_launch_each(lag, fp64):
         header = codec.L["gc"]
         assert np.array_equal(raw[0][:, :header], raw[1][:, :header]), k
     assert len(seen) == 17 and loops[0].batch.state()[2][:, 5].sum() == 1
+
+
+@pytest.mark.parametrize("which,own,fp64", [("pairs", False, False), ("pairs", True, False), ("plain", False, False),
+                                            ("plain", True, False), ("chain", False, False), ("chain", True, False),
+                                            ("pairs", True, True), ("plain", True, True), ("chain", True, True)])
+def test_servo_substeps_leave_the_blobs_of_a_launch_each(which, own, fp64):
+    """Every byte of the exported states, the contact lists with the entries
+    past their ends, drive channels and colours included, over falls and
+    curls in which contacts come and go within a call; `own`: masses,
+    friction and velocities per environment."""
+    if which == "chain":
+        text, home, feet, reach, curl = caterpillar(20, pairs=True), np.zeros(19), [1, 2], 1.2, 1.3
+    else:
+        text, meta = model_text(self_contact=which == "pairs")
+        home, reach, curl = np.array(meta["home"]), 0.6, 0.0
+        feet = [meta["body_names"].index(n) for n in ("left_foot", "right_foot")]
+    E, J, dtype, rng = 61, len(home), torch.float64 if fp64 else torch.float32, np.random.default_rng(17)
+    t = lambda a: torch.tensor(a, dtype=dtype, device=DEV)  # noqa: E731
+    root, ext = np.zeros((E, 6)), np.zeros((E, 5))
+    root[:, 2] = rng.uniform(0, 0.02, E)
+    root[:, 3:5] = rng.uniform(-0.2, 0.2, (E, 2))
+    ext[:, 0], ext[:, 1] = rng.uniform(0.3, 1, E), rng.uniform(0.9, 1.1, E)
+    ext[:, 2:] = rng.normal(0, 0.3, (E, 3))
+    q = home + rng.uniform(-curl, curl, (E, J))
+    loops = []
+    for _ in range(2):
+        b = CudaBatch.from_text(text, E, DT, ITER, 0, fp64)
+        b.reset(torch.ones(E, dtype=torch.bool, device=DEV), t(q), t(root), t(ext) if own else None)
+        loops.append(ServoLoop(b, servo_params(**SYNTHETIC_SUPPLY, lag=1), home, [0.0, 0.0, 0.01], feet=feet,
+                               foot_sites=[[0.01, 0.0, -0.006]] * 2))
+    shrunk = torch.zeros(2, dtype=torch.long)
+    for k in range(14):
+        targets, counts = t(home + rng.uniform(-reach, reach, (E, J))), []
+        loops[0].substeps(targets, 4)
+        loops[1].substeps(targets, 4, lambda loop: counts.append(loop.batch.contact_counts()))
+        raw = [x.batch.export_state() for x in loops]
+        assert torch.equal(raw[0], raw[1]), k
+        counts = torch.stack(counts)
+        shrunk += (counts.amax(0) > counts[-1]).sum(0).cpu()
+        if k == 6:  # another drive between: held controls, then a target launch
+            for x in loops:
+                x.batch.advance(1)
+                x.batch.step(targets, torch.zeros(E, 3, dtype=dtype, device=DEV), 1, 8.0, 0.0)
+    # lists that were longer within a call than at its end
+    assert shrunk[0] > 0 and (shrunk[1] > 0 or which != "pairs"), shrunk
