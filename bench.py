@@ -180,7 +180,7 @@ def host_facts():
 
 
 class MissingReference(RuntimeError):
-    """The reference's CPU build is not there (its sources are absent)."""
+    """The reference's CPU build was never made here (no built file)."""
 
 
 def cpu_baseline(model, home, seconds_budget=12.0):
@@ -199,16 +199,20 @@ def cpu_baseline(model, home, seconds_budget=12.0):
     port    the oracle's own threaded batch (oracle.OracleBatch, the same
             CpuBatch semantics over this repository's restatement) on the
             same workload and threads, for about a third of the budget.
-    The reference build is required: without oracle/_ref this raises."""
+    Without a build this raises MissingReference; a build that is there and
+    does not load raises its own error."""
     import json as _json
     import subprocess
 
     import numpy as np
 
-    sys.path.insert(0, str(ROOT / "oracle" / "_ref"))
+    ref = ROOT / "oracle" / "_ref"
+    sys.path.insert(0, str(ref))
     try:
         import _duck_reference
-    except ImportError as e:
+    except ModuleNotFoundError as e:
+        if e.name != "_duck_reference" or any(ref.glob("_duck_reference*")):
+            raise
         raise MissingReference("the reference CPU build is missing (make -C oracle ref): "
                                f"{e}") from e
     facts = host_facts()
@@ -629,6 +633,7 @@ def main():
         try:
             line["cpu_baseline"] = cpu_baseline(model, home)
         except MissingReference as e:  # the GPU figures stand without it
+            line["cpu_baseline_missing"] = str(e)
             print(f"cpu_baseline: {e}", file=sys.stderr, flush=True)
     print(json.dumps(line), flush=True)
 

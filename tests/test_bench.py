@@ -35,6 +35,27 @@ def test_cpu_baseline_requires_the_reference_build(models, home, monkeypatch):
         bench.cpu_baseline(models["standing"], np.asarray(home), seconds_budget=0.1)
 
 
+def test_a_reference_build_that_does_not_load_is_no_missing_one(models, home, monkeypatch, tmp_path):
+    """A built file that cannot be imported, by its own error or by another
+    interpreter's name, fails the run instead of reading as an absent build."""
+    ref = tmp_path / "oracle" / "_ref"
+    ref.mkdir(parents=True)
+    monkeypatch.setattr(bench, "ROOT", tmp_path)
+    monkeypatch.setattr(sys, "path", [str(ref), *(p for p in sys.path if "_ref" not in p)])
+    monkeypatch.delitem(sys.modules, "_duck_reference", raising=False)
+    module = ref / "_duck_reference.py"
+    for text in ('raise ImportError("undefined symbol: x")', "import no_such_runtime_library"):
+        module.write_text(text)
+        with pytest.raises(ImportError) as failure:
+            bench.cpu_baseline(models["standing"], np.asarray(home), seconds_budget=0.1)
+        assert not isinstance(failure.value, bench.MissingReference)
+        monkeypatch.delitem(sys.modules, "_duck_reference", raising=False)
+    module.unlink()
+    (ref / "_duck_reference.cpython-27-x86_64-linux-gnu.so").touch()
+    with pytest.raises(ModuleNotFoundError):
+        bench.cpu_baseline(models["standing"], np.asarray(home), seconds_budget=0.1)
+
+
 def test_roofline_object_carries_bound_valu_and_occupancy():
     """The roofline of a bench line: the metric's HBM figures, the true bound
     (latency, not HBM), the FP32-VALU fraction from the recorded op counts of
