@@ -54,6 +54,9 @@ ENVS, DT, ITERATIONS, KP = 4096, 0.005, 10, 8.0
 BOUND = ("latency: one wave per SIMD (the LDS each workgroup stages allows no second), "
          "whose dependent FP32 VALU chain and LDS round trips set the step time; neither "
          "HBM- nor MFMA-bound (profiles/advance_kernel_microduck_4096_counters.md)")
+BOUND_DENSE = ("issue: two waves per SIMD (the dense step), whose VALU instructions fill most of "
+               "the issue slots; neither HBM- nor MFMA-bound "
+               "(profiles/dense_kernel_drop_16384.md, profiles/rollout_32768.md)")
 
 
 def state_bytes_per_env(contacts, bodies=15, joints=14):
@@ -76,18 +79,20 @@ def algorithmic_bytes_per_launch(envs, contacts, model_bytes, self_contacts=0.0)
     return envs * per_env + model_bytes
 
 
-def servo_bytes_per_env(contacts, self_contacts, joints=14, feet=2):
-    """One fused servo substep of one env: the persistent state read and
-    written once, plus the actuator's buffers -- the ring slot written and the
-    delayed one read, the targets and root offset read, previous raw/applied
-    torques read and written, the motor channels and supply written, the
-    self-contact maxima read and written, the refresh outputs written (root
-    gravity, angular, linear and origin velocity; per foot the force, site
-    position and velocity) and the air/contact timers read and written."""
+def servo_bytes_per_env(contacts, self_contacts, joints=14, feet=2, substeps=1):
+    """One launch of `substeps` fused servo substeps of one env.  Once: the
+    persistent state read and written, and the targets, root offset, previous
+    raw and applied torques and the initialized flag read.  Every substep: the
+    ring slot written and the delayed one read, the previous torques, motor
+    channels and supply written, the self-contact maxima and the air/contact
+    timers read and written, the refresh outputs (root gravity, angular,
+    linear and origin velocity; per foot the force, site position and
+    velocity) and the flag written."""
     state = 2 * (state_bytes_per_env(contacts) + SELF_CONTACT_BYTES * self_contacts)
-    actuator = (2 * joints + joints + 3 + 2 * 2 * joints + 3 * joints + 1 + 2 * 2
-                + 4 * 3 + feet * 9 + 2 * 2 * feet) * 4 + 2  # + the initialized flag R/W
-    return state + actuator
+    inputs = (joints + 3 + 2 * joints) * 4 + 1
+    substep = (2 * joints + 2 * joints + 3 * joints + 1 + 2 * 2 + 2 * 2 * feet
+               + 4 * 3 + feet * 9) * 4 + 1
+    return state + inputs + substeps * substep
 
 
 def measured_traffic():
@@ -127,13 +132,16 @@ def flop_per_env_step(workload):
 
 
 def roofline(kernel_s, algo_bytes, env_steps_per_launch, flop_workload, occupancy,
-             traffic=None, kernel="advanceKernel"):
+             traffic=None, kernel=None):
     """The roofline object of a bench line for the dominant kernel: HBM
-    (the metric's figures), the FP32-VALU fraction and the occupancy."""
+    (the metric's figures), the FP32-VALU fraction and the occupancy, which
+    tells the step of two waves per SIMD from the full one."""
     achieved = algo_bytes / kernel_s / 1e9
+    dense = bool(occupancy) and occupancy.get("waves_per_simd", 0) >= 2
+    kernel = kernel or ("denseKernel" if dense else "advanceKernel")
     out = {
-        "bound": "latency",
-        "bound_detail": BOUND,
+        "bound": "issue" if dense else "latency",
+        "bound_detail": BOUND_DENSE if dense else BOUND,
         "achieved": achieved,
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
@@ -422,11 +430,13 @@ def other_workload(args):
             torch.cuda.synchronize()
             timing[fused] = time.perf_counter() - t0
             if fused:
-                kernel_s = begin.elapsed_time(end) / 1000.0 / (args.steps * substeps)
+                # one launch per control step
+                kernel_s = begin.elapsed_time(end) / 1000.0 / args.steps
                 counts = batch.contact_counts().float().mean(0)
-                algo = E * servo_bytes_per_env(float(counts[0]), float(counts[1])) + 4 * 4096
-                line_roofline = roofline(kernel_s, algo, E, "servo",
-                                         batch.kernel_info("servo_substep"),
+                algo = E * servo_bytes_per_env(float(counts[0]), float(counts[1]),
+                                               substeps=substeps) + 4 * 4096
+                line_roofline = roofline(kernel_s, algo, E * substeps, "servo",
+                                         batch.kernel_info("servo_substeps"),
                                          kernel="servoStepKernel")
         wall = timing[True]
         value = E * args.steps * substeps / wall
@@ -435,7 +445,7 @@ def other_workload(args):
                               "load-dependent friction, servo targets HOME + U(-0.3, 0.3) per "
                               "control step, body contacts between the leg chains, refresh "
                               "quantities (root frame, foot forces and sites, timers) per "
-                              "substep; one launch per substep",
+                              "substep; one launch per control step",
                   "envs": E, "iterations": ITERATIONS, "dt_s": DT,
                   "physics_steps_per_control_step": substeps,
                   "unfused_env_steps_per_s": E * args.steps * substeps / timing[False],

@@ -78,6 +78,29 @@ def test_roofline_object_carries_bound_valu_and_occupancy():
     assert bench.roofline(1e-4, 1e6, 1, "no-such-workload", None)["valu"] is None
 
 
+def test_roofline_object_tells_the_dense_step():
+    dense = bench.roofline(1e-4, 1e6, 1, "drop", {"waves_per_simd": 2.0})
+    assert dense["kernel"] == "denseKernel" and dense["bound"] == "issue"
+    assert "two waves per SIMD" in dense["bound_detail"]
+    full = bench.roofline(1e-4, 1e6, 1, "sweep", {"waves_per_simd": 1.0})
+    assert full["kernel"] == "advanceKernel" and "one wave per SIMD" in full["bound_detail"]
+    named = bench.roofline(1e-4, 1e6, 1, "home", {"waves_per_simd": 2.0}, kernel="control step")
+    assert named["kernel"] == "control step" and named["bound"] == "issue"
+    for line in (dense, full):
+        for name in bench.re.findall(r"profiles/\S+\.md", line["bound_detail"]):
+            assert (ROOT / name).is_file()
+
+
+def test_servo_bytes_of_a_launch_count_the_state_once():
+    """Substeps of one launch add their outputs, not another state and input
+    read: the targets, root offset, torques and the flag come once."""
+    one, four = (bench.servo_bytes_per_env(8, 1, substeps=n) for n in (1, 4))
+    once = 2 * (bench.state_bytes_per_env(8) + 68) + (14 + 3 + 28) * 4 + 1
+    assert four - once == 4 * (one - once)
+    assert one - once == (28 + 28 + 42 + 1 + 4 + 8 + 12 + 18) * 4 + 1
+    assert one == bench.servo_bytes_per_env(8, 1)
+
+
 def test_servo_bytes_count_the_actuator_buffers():
     plain = 2 * bench.state_bytes_per_env(8)
     assert bench.servo_bytes_per_env(8, 0) > plain
