@@ -308,19 +308,22 @@ class Batch final : public BatchBase {
   // Environments a wave of the full step advances in a launch of n.  The
   // environments of a wave take each other's turns (contact rounds, body-pair
   // queries, third colours, the double step's angle branches), so they get
-  // waves of their own while the launch stays within a quarter of the waves
-  // that the device holds at once: a process has four hardware queues, so the
-  // launches of as many streams still run side by side.  Past that line they
-  // take turns, which costs more than the own waves give one launch alone
-  // (MicroDuck in double, us per step: two batches of 500 as 125 waves each
-  // 323, as 500 waves 568; three of 250 as 125 waves 303, as 250 waves 433;
-  // alone, 500 as 125, 250 and 500 waves 338, 319 and 296).  For float that
-  // quarter is one wave per compute unit, where waves begin to cost each other
-  // LDS turns anyway (a sweep of 100 as 100, 50 and 25 waves: 135, 139, 143).
+  // waves of their own while the launch stays within a share of the waves that
+  // the device holds at once: the launches of other streams run beside it, and
+  // past the shares they take turns.  A quarter (four hardware queues a
+  // process): for float that is one wave per compute unit, where waves begin to
+  // cost each other LDS turns anyway (a sweep of 100 as 100, 50 and 25 waves:
+  // 135, 139, 143 us), and the split double solve gains nothing past it (250
+  // environments as 63, 125 and 250 waves: 245, 241, 241).  Four environments
+  // with one lane per block solve wait for each other most, so those launches
+  // take half: us per step of 500 MicroDuck environments in double as 125, 250
+  // and 500 waves, alone 338, 316, 296, two batches on two streams 323, 298,
+  // 568, three 304, 432, 852.  (Two to a wave, the generic state: 100 chains of
+  // 24 as 50 and 100 waves, alone 438 and 416, three batches 415 and 503.)
   static constexpr int kResident = // workgroups of a compute unit's LDS
       int(160 * 1024 / (sizeof(Frames<R, B, J>) + G * sizeof(typename Stepper<R, B, J, CG, CS, L, PL>::Env)));
   int perWave(int n) const {
-    const int waves = cus * kResident / 4;
+    const int waves = cus * kResident / (PL == 1 && L == 16 ? 2 : 4);
     int per = 1;
     while (per < G && (n + per - 1) / per > waves)
       per *= 2;
