@@ -633,9 +633,6 @@ template <class R, int B, int J, int CG, int CS, int L, class Env>
 __device__ __forceinline__ void servoEpilogue(const ServoArgs<R> &sv, const DeviceModel<R> &M, Env &E,
                                               int e, int lane);
 
-// Per-launch step: controls, `substeps` physics steps, write-back; with
-// Servo, the controls are the motor channels of one servo substep and the
-// launch ends with the substep's statistics and refresh quantities.
 // The model's solve-time view (Frames), built once per batch by framesKernel
 // into device memory; every workgroup of a step copies it into LDS whole (one
 // round of loads instead of a round trip per field).  Thread t of T.
@@ -717,8 +714,9 @@ __global__ void framesKernel(const DeviceModel<R> *model, Frames<R, B, J> *out) 
   stageFrames<R, B, J>(*out, *model, threadIdx.x, blockDim.x);
 }
 
-//
-// `block` is the wave's number: it advances environments block * per + g,
+// A launch of one wave: controls, `substeps` physics steps, write-back; with
+// Servo, the controls are the motor channels of a servo substep, which ends
+// with its statistics and refresh quantities.  `block` is the wave's number: it advances environments block * per + g,
 // with per = args.perWave <= G (Dense: G).
 // Dense: the step of target controls of a model without body pairs with two
 // waves per SIMD -- kDenseWaves waves per workgroup, each on its own (they
@@ -2018,14 +2016,15 @@ __global__ __launch_bounds__(64) __attribute__((aligned(32768))) void advanceKer
 }
 
 // The step of a batch with more waves than SIMDs (stepBody's Dense).  The full
-// step's wave issues VALU work in 59 % of its life and its 40 KiB of LDS and
+// step's wave issues VALU work in 62 % of its life and its 40 KiB of LDS and
 // 400 registers admit no second one beside it, so such a batch ran in rounds;
 // here two waves share a SIMD (20 KiB and 256 registers each) and fill each
-// other's waits: VALU issue 85 % of the time, a wave's life 47.6 k -> 66.5 k
-// quad-cycles at 32768 standing environments.  Four steps of them: 2470 ->
-// 1854 us; the landed drop of 16384: 488 -> 379 us.  What is left is the issue
-// of its 27.3 k VALU instructions, and the registers that detection spills
-// (keep() keeps addresses from being spilled across the iterations: without it
+// other's waits: VALU issue 88 % of the time, a wave's life 45.0 k -> 63.7 k
+// quad-cycles a step at 32768 environments of a rollout.  Four steps of them:
+// 2474 -> 1851 us; the landed drop of 16384: 481 -> 372 us.  What is left is
+// the issue of its 27.1 k VALU instructions a step, and the registers that
+// detection spills (564 B per lane, 202 MB more writes a launch of the drop;
+// keep() keeps addresses from being spilled across the iterations: without it
 // 2233 us).
 template <class R, int B, int J, int CG, int CS, int L, int PL = defaultSolveLanes(L)>
 __global__ __launch_bounds__(64 * kDenseWaves, 2) __attribute__((aligned(32768))) void denseKernel(StepArgs args) {

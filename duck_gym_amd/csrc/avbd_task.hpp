@@ -448,7 +448,7 @@ template <class R> __device__ __forceinline__ void waveLogs(R (&v)[kTaskLogs]) {
 // environments, in two launches: here a wave of 64 environments forms its
 // terms (the root's pose and velocity straight from the blobs) and their sums
 // and maxima as row 1 + block of `out`; taskLogReduceKernel folds the rows
-// into row 0 in row order, so the values do not depend on timing.  Bound by
+// into row 0 in a fixed order, so the values do not depend on timing.  Bound by
 // launch: 2 x 4 us at 4096 environments in the place of a state snapshot and
 // some 50 torch launches (about 190 us of them on the stream).
 template <class R, int B, int J, int CG, int CS>
