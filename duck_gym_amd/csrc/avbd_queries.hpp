@@ -58,6 +58,21 @@ template <class R, int B, int J, int CG, int CS> struct StateView {
     s.ngc = 0;
     s.nsc = 0;
   }
+  // Fails an imported state whose contact lists cannot be the model's (a count
+  // past the list's end, a body or shape that is not there), with its lists
+  // empty: every launch walks the lists by their counts and indexes by their
+  // ids, in the record and, in the dense step and the queries, in memory.
+  DUCK_HD void checkContacts() {
+    bool ok = s.ngc >= 0 && s.ngc <= CG && s.nsc >= 0 && s.nsc <= CS;
+    for (int i = 0; ok && i < s.ngc; ++i)
+      ok = gcBody(s.gc[i].id) < M.nb && gcShape(s.gc[i].id) < M.ns;
+    for (int i = 0; ok && i < s.nsc; ++i)
+      ok = scBody(s.sc[i].id) < M.nb && scOther(s.sc[i].id) < M.nb;
+    if (!ok) {
+      s.failed = 1;
+      s.ngc = s.nsc = 0;
+    }
+  }
   // Clears the claims of `drive` and `modelColours` that the blob's bytes do
   // not bear out (an imported state); keeps every true one, so that an export
   // and import of the same batch's state is the identity.
@@ -100,12 +115,13 @@ __global__ void initializeKernel(const DeviceModel<R> *model, unsigned char *sta
 }
 
 template <class R, int B, int J, int CG, int CS>
-__global__ void checkStampsKernel(const DeviceModel<R> *model, unsigned char *states,
+__global__ void checkImportKernel(const DeviceModel<R> *model, unsigned char *states,
                                   long long blobBytes, int count) {
   int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= count)
     return;
   StateView<R, B, J, CG, CS> v{*model, blobAt<EnvState<R, B, J, CG, CS>>(states, blobBytes, e)};
+  v.checkContacts();
   v.checkStamps();
 }
 

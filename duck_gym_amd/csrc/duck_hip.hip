@@ -771,8 +771,8 @@ public:
     wait(s);
     hipCheck(hipMemcpyAsync(dStates, src, size_t(blobBytes) * count, hipMemcpyDeviceToDevice, s),
              "import_state");
-    checkStampsKernel<R, B, J, CG, CS><<<blocks64(count), 64, 0, s>>>(dModel, dStates, blobBytes, count);
-    launched("checkStampsKernel");
+    checkImportKernel<R, B, J, CG, CS><<<blocks64(count), 64, 0, s>>>(dModel, dStates, blobBytes, count);
+    launched("checkImportKernel");
     customBodies = true;
     record(s);
   }

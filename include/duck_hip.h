@@ -151,7 +151,9 @@ long long duck_state_bytes(void *handle);
  * offset of sc, self-contact bytes, then the field offsets of a ground contact
  * (id local anchor c0 lambda penalty) and of a self contact (id local localB
  * t1 t2 n c0 friction lambda penalty).  Export/import copy all E blobs
- * (E * duck_state_bytes bytes) to/from a device buffer. */
+ * (E * duck_state_bytes bytes) to/from a device buffer; an imported state whose
+ * contact lists cannot be the model's (a count out of range, an id of a body or
+ * shape that is not there) fails, with empty lists. */
 int duck_state_layout(void *handle, long long *out);
 int duck_export_state(void *handle, void *dst, void *hip_stream);
 int duck_import_state(void *handle, const void *src, void *hip_stream);

@@ -80,3 +80,49 @@ def test_dense_step_is_the_full_step(which, custom):
     assert most >= contacts
     failed = batches[0].state()[2][:, 5]
     assert int(failed.sum()) == (2 if J else 0)
+
+
+@pytest.mark.parametrize("dense", [False, True])
+def test_imported_states_with_impossible_contact_lists_fail(dense):
+    """A count past the list's end or an id of no body or shape: the
+    environment fails with empty lists and stays as it was imported, in the
+    full and the dense step; the others step as if it were not there, and an
+    export imported again is itself."""
+    text, meta = model_text()
+    E = 4 * 4 * torch.cuda.get_device_properties(0).multi_processor_count + 5 if dense else 23
+    batches = [CudaBatch.from_text(text, E, DT, ITER) for _ in range(2)]
+    assert (batches[0].kernel_info()["waves_per_simd"] == 2) == dense
+    home = torch.tensor(np.tile(meta["home"], (E, 1)), dtype=torch.float32, device=DEV)
+    zero = torch.zeros(E, 6, device=DEV)
+    for b in batches:
+        b.reset(torch.ones(E, dtype=torch.bool, device=DEV), home, zero)
+        for _ in range(3):
+            b.step(home, zero[:, :3].contiguous(), 1, 8.0, 0.0)
+    raw = batches[0].export_state()
+    batches[0].import_state(raw)
+    assert torch.equal(batches[0].export_state(), raw)
+    L, host = batches[0].codec().L, raw.cpu().numpy()
+    ints = lambda e, at: host[e, at:at + 4].view(np.int32)  # noqa: E731
+    assert ints(0, L["ngc"])[0] > 1
+    body, shape = int(batches[0].num_bodies), 63
+    bad = {1: ("ngc", L["CG"] + 1), 4: ("ngc", -1), 6: ("ngc", 2**30), 9: ("nsc", L["CS"] + 1), 11: ("nsc", -7),
+           13: ("body", body << 6), 17: ("shape", shape), 22: ("ngc", 2**31 - 1)}
+    for e, (what, value) in bad.items():
+        if what in ("ngc", "nsc"):
+            ints(e, L[what])[:] = value
+        else:
+            ints(e, L["gc"] + L["gcBytes"] + L["gc_id"])[:] = value
+    batches[0].import_state(torch.tensor(host, device=DEV))
+    imported = batches[0].state()[0]
+    for b in batches:
+        b.step(home, zero[:, :3].contiguous(), 2, 8.0, 0.0)
+        b.advance(1)
+    bodies, _, diag = batches[0].state()
+    failed = torch.zeros(E, dtype=torch.bool, device=DEV)
+    failed[list(bad)] = True
+    assert torch.equal(diag[:, 5] != 0, failed)
+    assert torch.equal(bodies[failed], imported[failed])
+    assert int(batches[0].contact_counts()[failed].sum()) == 0
+    assert int(batches[0].contact_forces()[failed].count_nonzero()) == 0
+    assert torch.equal(bodies[~failed], batches[1].state()[0][~failed])
+    assert torch.equal(batches[0].export_state()[~failed], batches[1].export_state()[~failed])
