@@ -197,7 +197,7 @@ def cpu_baseline(model, home, seconds_budget=12.0):
     batch   kernel.cuh's CPU batch (CpuBatch32, src/cuda/cpu_bindings.cpp,
             compiled in place into oracle/_ref) on the same 4096-env workload,
             env-striped over every CPU this process may use (capped by
-            OMP_NUM_THREADS where set: a GPU box grants 16 per GPU), for about
+            OMP_NUM_THREADS where set), for about
             `seconds_budget` seconds;
     single  one env in float64 on one thread for 200 steps (CpuBatch64),
             timed around step() only, as src/main.cpp:63-68 times its solver;
